@@ -374,8 +374,9 @@ def tolerance(case):
     if kind == "noise":
         # one fp32 ulp of the normal's formula, or (bf16) a rounding that falls the other way
         return {"rel": 1e-6} if case["dtype"] == "float32" else {"rel": 1e-3}
-    # bf16 results of fp32 arithmetic: about four times the distance from the 64-bit result
-    return {"rel": {"norm": 7e-3, "guide": 1.2e-2, "ffn": 1.2e-2, "te": 4e-2, "model": 3e-2}.get(kind, 1.6e-2)}
+    # four times the measured distance of the bf16 results from the 64-bit ones: norm 0.0024, guide 0.009, ffn 0.003,
+    # te 0.0056, model 0.0095, an attention layer 0.0069 to 0.0093
+    return {"rel": {"norm": 1e-2, "guide": 3.6e-2, "ffn": 1.2e-2, "te": 2.3e-2, "model": 4e-2}.get(kind, 3.6e-2)}
 
 
 # --------------------------------------------------------------------------------------------------------------------
