@@ -353,6 +353,29 @@ int ltxk_attn_combine(void *out, const void *part, int64_t part_bstride, int64_t
                       int64_t lse_cstride, int64_t lse_hstride, int64_t lse_tstride, const void *logits,
                       int64_t batch, int64_t parts, int64_t tokens, int64_t heads, int64_t head_dim, void *stream);
 
+/* Bytes of workspace ltxk_attention needs for this shape: 0 unless the keys are
+ * cut into parts (few query tiles over many keys). */
+int64_t ltxk_attention_workspace_bytes(int64_t batch, int64_t tokens_q, int64_t tokens_k, int64_t heads,
+                                       int64_t head_dim);
+
+/* Softmax attention with the head merge and the per-head gate, heads of 64 or
+ * 128, no mask:
+ *   o[b, t, h, :]        = round(sum_j softmax_j(scale * q[b, t, h].k[b, j, h]) v[b, j, h, :])
+ *   out[b*Tq + t, h, :]  = round(o * 2*sigmoid(logits[b*Tq + t, h]))  (o if logits NULL)
+ * q is bf16 at q + b*q_bstride + t*q_tstride + h*head_dim (elements, multiples
+ * of 8, token strides at least heads*head_dim), k and v likewise; out is
+ * contiguous token-major [batch*tokens_q, heads*head_dim], logits contiguous
+ * [batch*tokens_q, heads].  Scores, softmax and sums are fp32, the weights
+ * bf16 in the product with v.  The keys of one batch item span less than 2^31
+ * bytes.  `workspace`: device memory of ltxk_attention_workspace_bytes, 16-byte
+ * aligned (NULL if that is 0), in use until the call's work has run.
+ * Replaces SDPA, the head merge and the gate (standalone/ltx_nn.py:22-26,
+ * 227-235). */
+int ltxk_attention(void *out, const void *q, int64_t q_bstride, int64_t q_tstride, const void *k, int64_t k_bstride,
+                   int64_t k_tstride, const void *v, int64_t v_bstride, int64_t v_tstride, const void *logits,
+                   int64_t batch, int64_t tokens_q, int64_t tokens_k, int64_t heads, int64_t head_dim, float scale,
+                   void *workspace, int64_t workspace_bytes, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

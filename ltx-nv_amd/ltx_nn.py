@@ -4,10 +4,10 @@
 Kept as in the reference (names, signatures, shapes): rms_norm, sdpa,
 generate_freq_grid_np/_pytorch, precompute_freqs_cis, apply_split_rotary_emb,
 TimestepEmbedder, CombinedTimestepEmbeddings, AdaLayerNormSingle, Attention,
-FeedForward.  Linear layers and scaled-dot-product attention stay on
-PyTorch-ROCm; RMSNorm, q/k norm + split RoPE, the per-head gate and
-GELU-tanh are ltxk kernels, with fp32 arithmetic and one bf16 rounding per
-output.
+FeedForward.  Linear layers stay on PyTorch-ROCm; RMSNorm, q/k norm + split
+RoPE, unmasked attention with the per-head gate and GELU-tanh are ltxk kernels,
+with fp32 arithmetic and one bf16 rounding per output.  `sdpa` and masked
+attention are PyTorch-ROCm's.
 """
 
 import functools
@@ -73,6 +73,21 @@ def key_split_partials(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, parts:
     qc = q.unsqueeze(1).expand(b, parts, h, tq, d).reshape(b * parts, h, tq, d)
     out, lse = torch.ops.aten._scaled_dot_product_flash_attention(qc, chunks(k), chunks(v))[:2]
     return out, lse
+
+
+def fused_attention_applies(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, heads: int, dim_head: int) -> bool:
+    """Whether unmasked attention of token-major q over k, v runs on
+    ltxk_attention: contiguous 16-byte aligned bf16 tensors on one ROCm device,
+    heads of 64 or 128, keys of one batch item within the kernel's 32-bit
+    offsets, and no gradient to record."""
+    if not (dim_head in ltxk.ATTENTION_HEAD_DIMS and q.ndim == k.ndim == 3 and v.shape == k.shape
+            and q.shape[0] == k.shape[0] and q.shape[2] == k.shape[2] == heads * dim_head and k.shape[1] > 0
+            and (k.shape[1] + 64) * k.shape[2] < 2**30):
+        return False
+    if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):
+        return False
+    return all(t.is_cuda and t.device == q.device and t.dtype == torch.bfloat16 and t.is_contiguous()
+               and t.data_ptr() % 16 == 0 for t in (q, k, v))
 
 
 # ---------------------------------------------------------------------------
@@ -278,10 +293,10 @@ class AdaLayerNormSingle(torch.nn.Module):
 class Attention(torch.nn.Module):
     """Multi-head attention with RMS q/k-norm, split RoPE and per-head gating (ltx_nn.py:166-236).
 
-    q/k/v projections and SDPA are PyTorch-ROCm.  q_norm/k_norm + RoPE run as
-    one in-place ltxk_qk_norm_rope launch on the fresh projections; the head
-    merge, the perturbation blend (B=4 guidance batch) and the per-head
-    2*sigmoid gate are one ltxk_head_gate pass over the attention output.
+    q/k/v projections are PyTorch-ROCm.  q_norm/k_norm + RoPE run as one
+    in-place ltxk_qk_norm_rope launch on the fresh projections; attention, the
+    head merge and the per-head 2*sigmoid gate are one ltxk_attention call
+    (`attend`).
     """
 
     def __init__(self, query_dim: int, context_dim: int | None = None, heads: int = 8, dim_head: int = 64,
@@ -323,12 +338,22 @@ class Attention(torch.nn.Module):
 
     def attend(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gates: torch.Tensor | None,
                mask: torch.Tensor | None = None, perturbation_mask: torch.Tensor | None = None) -> torch.Tensor:
-        """The part of forward after q/k norm + RoPE (ltx_nn.py:219-236): SDPA on
-        token-major q, k, v (B, T, H*Dh), the head merge [+ perturbation blend]
-        [+ per-head gate] in one ltxk_head_gate pass, then to_out.  Lets a caller
-        prepare the q/k of two attentions in one launch (Block's A2V/V2A)."""
+        """The part of forward after q/k norm + RoPE (ltx_nn.py:219-236): attention
+        on token-major q, k, v (B, T, H*Dh), the head merge [+ perturbation blend]
+        [+ per-head gate], then to_out.  Without a mask and for heads of 64 or 128
+        that is ltxk_attention with the gate inside it (the blend as an
+        ltxk_head_gate pass after it); otherwise torch's SDPA, then ltxk_head_gate.
+        Lets a caller prepare the q/k of two attentions in one launch (Block's
+        A2V/V2A)."""
         b = q.shape[0]
         h, dh = self.heads, self.dim_head
+        pm = None
+        if perturbation_mask is not None:
+            pm = perturbation_mask.reshape(-1).to(torch.bfloat16).contiguous()
+        if mask is None and fused_attention_applies(q, k, v, h, dh):
+            if pm is None:
+                return self.to_out(ltxk.attention(q, k, v, h, gates))
+            return self.to_out(ltxk.head_gate(ltxk.attention(q, k, v, h), gates, v=v, mask=pm, heads=h))
         q4 = q.view(b, -1, h, dh).transpose(1, 2)
         k4 = k.view(b, -1, h, dh).transpose(1, 2)
         v4 = v.view(b, -1, h, dh).transpose(1, 2)
@@ -346,9 +371,6 @@ class Attention(torch.nn.Module):
             out = attn.transpose(1, 2).reshape(b, -1, h * dh)
         else:
             # head merge [+ perturbation blend] [+ per-head gate] in one pass
-            pm = None
-            if perturbation_mask is not None:
-                pm = perturbation_mask.reshape(-1).to(torch.bfloat16).contiguous()
             out = ltxk.head_gate(attn, gates, v=v.contiguous() if pm is not None else None, mask=pm)
         return self.to_out(out)
 

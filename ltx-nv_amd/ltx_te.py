@@ -126,8 +126,10 @@ class Embeddings1DConnector(torch.nn.Module):
             additive_mask = torch.zeros_like(additive_mask)
         pe = self._rope(b, s, hidden_states.device, hidden_states.dtype)
         x, pending = hidden_states.contiguous(), None
+        # a mask of zeros adds nothing to the scores: the blocks run unmasked
+        mask = None if self.num_registers else additive_mask
         for block in self.blocks:
-            x, pending = block._run(x, pending, additive_mask, pe, defer=True)
+            x, pending = block._run(x, pending, mask, pe, defer=True)
         if pending is None:
             return ltxk.rms_norm(x, None, 1e-6), additive_mask
         _, out = ltxk.add_norm_modulate(x, pending, eps=1e-6)  # last residual + the output norm

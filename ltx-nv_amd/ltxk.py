@@ -119,6 +119,12 @@ SIGNATURES = {
         [_c_vp, _c_vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_vp, _c_i64, _c_i64,
          _c_i64, _c_i64, _c_i64, _c_vp],
     ),
+    "ltxk_attention_workspace_bytes": (_c_i64, [_c_i64] * 5),
+    "ltxk_attention": (
+        _c_int,
+        [_c_vp, _c_vp, _c_i64, _c_i64, _c_vp, _c_i64, _c_i64, _c_vp, _c_i64, _c_i64, _c_vp, _c_i64, _c_i64, _c_i64,
+         _c_i64, _c_i64, _c_float, _c_vp, _c_i64, _c_vp],
+    ),
 }
 
 _lib = None
@@ -775,6 +781,37 @@ def attn_combine(part: torch.Tensor, lse: torch.Tensor, parts: int, logits: torc
     rc = load().ltxk_attn_combine(_ptr(out), _ptr(part), parts * ps[0], ps[0], ps[1], ps[2], _ptr(lse),
                                   parts * ls[0], ls[0], ls[1], ls[2], _ptr(logits), b, parts, t, h, dh, _stream(part))
     _check_rc(rc, "attn_combine")
+    return out
+
+
+ATTENTION_HEAD_DIMS = (64, 128)
+
+
+def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, heads: int, logits: torch.Tensor | None = None,
+              out: torch.Tensor | None = None) -> torch.Tensor:
+    """softmax(q k^T / sqrt(Dh)) v on token-major q (B, Tq, H*Dh), k and v (B, Tk, H*Dh), heads of 64 or 128,
+    gated per head by 2*sigmoid(logits (B, Tq, H)) when logits is given.  Returns (B, Tq, H*Dh)."""
+    b, tq, d = _btd(q, "q")
+    kb, tk, kd = _btd(k, "k")
+    _dev(v, "v")
+    if (kb, kd) != (b, d) or v.shape != k.shape:
+        raise ValueError(f"q {tuple(q.shape)}, k {tuple(k.shape)} and v {tuple(v.shape)} do not match")
+    dh = d // heads
+    if d != heads * dh or dh not in ATTENTION_HEAD_DIMS:
+        raise ValueError(f"width {d} is not {heads} heads of 64 or 128")
+    if logits is not None:
+        _dev(logits, "logits")
+        if tuple(logits.shape) != (b, tq, heads):
+            raise ValueError(f"logits {tuple(logits.shape)} != {(b, tq, heads)}")
+    out = _out_like(out, q)
+    if out.numel() == 0:
+        return out
+    lib = load()
+    nbytes = lib.ltxk_attention_workspace_bytes(b, tq, tk, heads, dh)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes else None
+    rc = lib.ltxk_attention(_ptr(out), q.data_ptr(), tq * d, d, k.data_ptr(), tk * d, d, v.data_ptr(), tk * d, d,
+                            _ptr(logits), b, tq, tk, heads, dh, dh ** -0.5, _ptr(ws), nbytes, _stream(q))
+    _check_rc(rc, "attention")
     return out
 
 

@@ -1,0 +1,92 @@
+"""ltxk_attention (csrc/flash.hip) against softmax attention in fp64 (GPU), at the
+edges of its query and key tiles, where its launches are cut over the keys, and
+on inputs whose first key tile weighs nothing."""
+
+import ctypes
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda")
+
+
+def _check(q, k, v, h, logits, got):
+    """Element by element: rounding to bf16 (8 significant bits) moves a value by at
+    most 2^-8 of it, so the weights' roundings move the result by at most
+    2^-8 sum_j w_j |v_j|, the output's and the gated output's by 2^-8 of their
+    value each; the fp32 sums and exponentials are far below that (2 %)."""
+    b, tq, d = q.shape
+    dh = d // h
+    for i in range(b):
+        for j in range(h):
+            c = slice(j * dh, (j + 1) * dh)
+            w = torch.softmax(q[i, :, c].double() @ k[i, :, c].double().T / math.sqrt(dh), -1)
+            want, spread = w @ v[i, :, c].double(), w @ v[i, :, c].double().abs()
+            bound = spread * 2.0**-8 + want.abs() * 2.0**-8
+            if logits is not None:
+                gate = 2 * torch.sigmoid(logits[i, :, j].double()).unsqueeze(-1)
+                want, bound = want * gate, (bound + want.abs() * 2.0**-8) * gate
+            err = (got[i, :, c].double() - want).abs()
+            assert bool((err <= bound * 1.02 + 1e-6).all()), f"item {i} head {j}: {(err / (bound + 1e-6)).max().item():.3f}"
+
+
+@pytest.mark.parametrize("b,tq,tk,h,dh,gated,spread", [
+    (1, 1, 1, 2, 64, True, 1.0), (1, 128, 64, 1, 128, False, 1.0), (2, 129, 65, 3, 64, True, 1.0),
+    (1, 127, 63, 2, 128, True, 3.0), (3, 257, 191, 3, 128, True, 1.5), (1, 33, 1000, 2, 64, True, 1.5),
+    (1, 5, 4099, 9, 128, True, 1.5), (4, 126, 2050, 2, 64, False, 3.0), (1, 8257, 520, 8, 64, True, 1.5),
+    (1, 8200, 600, 9, 128, True, 1.5)])
+def test_attention_matches_fp64(b, tq, tk, h, dh, gated, spread):
+    import ltxk
+
+    g = torch.Generator(device=DEV).manual_seed(tq * 7 + tk)
+    q, k, v = ((torch.randn(b, t, h * dh, device=DEV, generator=g) * s).to(torch.bfloat16)
+               for t, s in ((tq, spread), (tk, spread), (tk, 1.0)))
+    logits = torch.randn(b, tq, h, device=DEV, generator=g).to(torch.bfloat16) if gated else None
+    _check(q, k, v, h, logits, ltxk.attention(q, k, v, h, logits))
+
+
+@pytest.mark.parametrize("tk", [200, 2048])
+def test_first_tile_without_weight(tk):
+    """Scores of -inf over the whole first key tile (and, with the keys cut, over
+    a whole unit) weigh nothing; the other keys' softmax is unaffected."""
+    import ltxk
+
+    g = torch.Generator(device=DEV).manual_seed(5)
+    q = torch.rand(1, 40, 128, device=DEV, generator=g).to(torch.bfloat16) + 0.5
+    k, v = (torch.randn(1, tk, 128, device=DEV, generator=g).to(torch.bfloat16) for _ in range(2))
+    closed = 64 if tk == 200 else 1024
+    k[:, :closed] = -float("inf")
+    got = ltxk.attention(q, k, v, 2)
+    _check(q, k[:, closed:].contiguous(), v[:, closed:].contiguous(), 2, None, got)
+
+
+def test_strided_operands_and_refusals():
+    """q, k and v as columns of one wider buffer through the C entry equal the
+    contiguous call bit for bit; a stride that does not cover the heads, a head
+    of 96 and a missing workspace are refused."""
+    import ltxk
+
+    lib = ltxk.load()
+    b, t, h, dh = 2, 300, 2, 64
+    d = h * dh
+    qkv = torch.randn(b, t, 3 * d, device=DEV).to(torch.bfloat16)
+    q, k, v = (qkv[..., i * d:(i + 1) * d].contiguous() for i in range(3))
+    want = ltxk.attention(q, k, v, h)
+    out = torch.empty_like(want)
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    p, row = qkv.data_ptr(), 3 * d
+
+    def call(tstride=row, head_dim=dh, tk=t, nbytes=0):
+        return lib.ltxk_attention(out.data_ptr(), p, t * row, tstride, p + 2 * d, t * row, row, p + 4 * d, t * row, row,
+                                  None, b, t, tk, h, head_dim, dh**-0.5, None, nbytes, st)
+
+    assert lib.ltxk_attention_workspace_bytes(b, t, t, h, dh) == 0
+    assert call() == 0
+    torch.cuda.synchronize()
+    assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+    assert call(tstride=64) == ltxk.E_ARG and call(tstride=row + 4) == ltxk.E_ALIGN
+    assert call(head_dim=96) == ltxk.E_ARG and call(tk=0) == ltxk.E_ARG
+    assert lib.ltxk_attention_workspace_bytes(b, t, 4096, h, dh) > 0
+    assert call(tk=4096) == ltxk.E_ARG
