@@ -22,11 +22,15 @@
 //   and its weights are already the second product's operand.
 // * V is read from LDS by transposing reads, so neither operand is rearranged.
 // * The second product of a tile and the scores of the next run as one stream,
-//   LDS fragments four ahead: 592-602 us with the products apart.
+//   LDS fragments four ahead: 592-602 us with the products apart.  The loads of the
+//   next tile go between the products: 612 against 623 us (one box) with all of
+//   them ahead of the stream, and without any loads (a timing copy) 11 % less.
 // * The running maximum is exact in every tile.  Letting it lag up to 2^8 saves
 //   2-4 %, but then a row's largest weight is no longer exactly 1 and its
 //   rounding shows: relative error 2.26e-3 against 1.87e-3 (torch's 1.87e-3).
 #include "ltxk_common.h"
+
+#include <type_traits>
 
 namespace ltxk {
 namespace {
@@ -81,23 +85,22 @@ __device__ __forceinline__ int v_pos(int row, int c)
 
 typedef __attribute__((address_space(3))) char lds_char;
 
-// One wave's share of a 64-row tile: each load instruction moves 64 lanes x 16
-// bytes straight into LDS.  Rows past the last key repeat it (their scores are
-// masked), so nothing outside the tensor is read.
+// Part j of a wave's share of a 64-row tile: one load instruction moves 64 lanes
+// x 16 bytes straight into LDS.  Rows past the last key repeat it (their scores
+// are masked), so nothing outside the tensor is read.
+template <int D>
+constexpr int kLoads = kKeys * D * 2 / 1024 / kWaves;  // load instructions of a wave for a tile
+
 template <int D, bool V>
-__device__ __forceinline__ void load_tile(rsrc_t r, char *lds, int first_row, int last_row, uint32_t stride, int wave,
-                                          int lane)
+__device__ __forceinline__ void load_part(rsrc_t r, char *lds, int j, int first_row, int last_row, uint32_t stride,
+                                          int wave, int lane)
 {
-    constexpr int rows_per = 1024 / (2 * D);  // rows one instruction covers
-    constexpr int n = kKeys / rows_per / kWaves;  // instructions per wave
-#pragma unroll
-    for (int j = 0; j < n; ++j) {
-        const int row = (wave * n + j) * rows_per + lane / (D / 8);
-        const int pos = lane % (D / 8);
-        const int c = V ? v_pos<D>(row, pos) : k_pos<D>(row, pos);  // the permutations are involutions
-        const uint32_t off = static_cast<uint32_t>(min(first_row + row, last_row)) * stride + c * 16;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_char *)(lds + (wave * n + j) * 1024), 16, off, 0, 0, 0);
-    }
+    const int at = wave * kLoads<D> + j;
+    const int row = at * (1024 / (2 * D)) + lane / (D / 8);
+    const int pos = lane % (D / 8);
+    const int c = V ? v_pos<D>(row, pos) : k_pos<D>(row, pos);  // the permutations are involutions
+    const uint32_t off = static_cast<uint32_t>(min(first_row + row, last_row)) * stride + c * 16;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_char *)(lds + at * 1024), 16, off, 0, 0, 0);
 }
 
 __device__ __forceinline__ bf16x8 cat(bf16x4 a, bf16x4 b)
@@ -158,13 +161,14 @@ __global__ void __launch_bounds__(kWaves * 64, 2) flash_kernel(FlashParams p)
     const rsrc_t kr = make_rsrc(p.k + b * p.kbs + head * D, static_cast<uint32_t>(last) * p.kts + 2 * D);
     const rsrc_t vr = make_rsrc(p.v + b * p.vbs + head * D, static_cast<uint32_t>(last) * p.vts + 2 * D);
 
-    auto load_k = [&](int i, char *dst) {
-        if (i < n) load_tile<D, false>(kr, dst, (t0 + i) * kKeys, last, p.kts, wave, lane);
+    auto load_k = [&](int i, int part, char *dst) {
+        load_part<D, false>(kr, dst, part, (t0 + i) * kKeys, last, p.kts, wave, lane);
     };
-    auto load_v = [&](int i, char *dst) {
-        if (i < n) load_tile<D, true>(vr, dst, (t0 + i) * kKeys, last, p.vts, wave, lane);
+    auto load_v = [&](int i, int part, char *dst) {
+        load_part<D, true>(vr, dst, part, (t0 + i) * kKeys, last, p.vts, wave, lane);
     };
-    load_k(0, k0);
+#pragma unroll
+    for (int c = 0; c < kLoads<D>; ++c) load_k(0, c, k0);
 
     // Queries: lane l holds query l % 32, elements 16 s + 8 (l/32) .. + 7.
     const int row = first + wave * 32 + l32;
@@ -210,37 +214,32 @@ __global__ void __launch_bounds__(kWaves * 64, 2) flash_kernel(FlashParams p)
         const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds4 *)(vt + v_off[m][1] + st * 32 * D));
         return cat(lo, hi);
     };
-    // Matrix phase of tile i: the product of tile i - 1's weights with V, then
-    // tile i's scores, one stream of products with the fragments read ahead of
-    // them; the loads of later tiles first.
-    auto products = [&](bool pv, bool qk, const char *vp, const char *kc) {
-        if (pv) {
-            bf16x8 vf[NV];
+    // Matrix phase: a run of the stream of products that a tile takes, the weights
+    // times V of the tile before (0 .. NV - 1), then its scores (NV .. NV + NK - 1),
+    // with the LDS fragments read ahead of them and `loads(j)` between them.
+    auto products = [&](auto from, auto to, const char *vp, const char *kc, auto loads)
+                        __attribute__((always_inline)) {
+        bf16x8 f[NV + NK];
+        auto frag = [&](int j) { f[j] = j < NV ? v_frag(vp, j) : k_frag(kc, j - NV); };
 #pragma unroll
-            for (int j = 0; j < kAhead; ++j) vf[j] = v_frag(vp, j);
+        for (int j = from; j < from + kAhead; ++j) frag(j);
 #pragma unroll
-            for (int j = 0; j < NV; ++j) {
-                if (j + kAhead < NV) vf[j + kAhead] = v_frag(vp, j + kAhead);
-                o[j % MT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[j], __builtin_bit_cast(bf16x8, w[j / MT]),
+        for (int j = from; j < to; ++j) {
+            if (j + kAhead < to) frag(j + kAhead);
+            loads(j - from);
+            if (j < NV) {
+                o[j % MT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[j], __builtin_bit_cast(bf16x8, w[j / MT]),
                                                                     o[j % MT], 0, 0, 0);
-                __builtin_amdgcn_sched_barrier(0);
+            } else {
+                const int i = j - NV;
+                s[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[j], qf[i >> 1], i < 2 ? f32x16{} : s[i & 1], 0, 0, 0);
             }
-        }
-        if (qk) {
-            bf16x8 kf[NK];
-#pragma unroll
-            for (int j = 0; j < kAhead; ++j) kf[j] = k_frag(kc, j);
-#pragma unroll
-            for (int j = 0; j < NK; ++j) {
-                if (j + kAhead < NK) kf[j + kAhead] = k_frag(kc, j + kAhead);
-                s[j & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[j], qf[j >> 1], j < 2 ? f32x16{} : s[j & 1], 0, 0, 0);
-                __builtin_amdgcn_sched_barrier(0);
-            }
+            __builtin_amdgcn_sched_barrier(0);
         }
     };
     // Vector phase of tile i: its maximum, the rescale of what was summed so far
     // if a row's maximum grew, its weights.
-    auto softmax = [&](int i) {
+    auto softmax = [&](int i) __attribute__((always_inline)) {
         if (i == n - 1) {  // keys past the last get weight zero
             const int valid = p.tk - (t0 + i) * kKeys;
             if (valid < kKeys)
@@ -282,23 +281,34 @@ __global__ void __launch_bounds__(kWaves * 64, 2) flash_kernel(FlashParams p)
         sum += part[0] + part[1];
     };
 
-    // Tile i: kc holds its keys, vp the values of tile i - 1.  Tile i + 1's keys
-    // and tile i's values load into the other buffers meanwhile.
-    auto tile = [&](int i, const char *kc, const char *vp, char *kn, char *vn) {
-        load_k(i + 1, kn);
-        load_v(i, vn);
-        __builtin_amdgcn_sched_barrier(0);
-        products(i > 0, true, vp, kc);
+    // Tile i: kc holds its keys, vp the values of tile i - 1.  Its values and the
+    // next tile's keys (the last tile's once more after the last) load into the
+    // other buffers between the products.
+    using std::integral_constant;
+    auto tile = [&](int i, auto from, const char *kc, const char *vp, char *kn, char *vn)
+                    __attribute__((always_inline)) {
+        constexpr int kEvery = from == 0 ? 3 : 2;
+        const int next = min(i + 1, n - 1);
+        products(from, integral_constant<int, NV + NK>{}, vp, kc, [&](int j) __attribute__((always_inline)) {
+            if (j % kEvery) return;
+            const int c = j / kEvery;
+            if (c < kLoads<D>)
+                load_v(i, c, vn);
+            else if (c < 2 * kLoads<D>)
+                load_k(next, c - kLoads<D>, kn);
+        });
         softmax(i);
         __builtin_amdgcn_sched_barrier(0);
         tile_barrier();
     };
+    constexpr integral_constant<int, 0> whole;
     tile_barrier();
-    for (int i = 0; i < n; i += 2) {
-        tile(i, k0, v1, k1, v0);
-        if (i + 1 < n) tile(i + 1, k1, v0, k0, v1);
+    tile(0, integral_constant<int, NV>{}, k0, v1, k1, v0);
+    for (int i = 1; i < n; i += 2) {
+        tile(i, whole, k1, v0, k0, v1);
+        if (i + 1 < n) tile(i + 1, whole, k0, v1, k1, v0);
     }
-    products(true, false, n & 1 ? v0 : v1, nullptr);
+    products(whole, integral_constant<int, NV>{}, n & 1 ? v0 : v1, nullptr, [](int) {});
 
     // Lane l: query l % 32, columns 32 m + 8 j + 4 half + (0..3) in registers 4 j ..
     const float total = pair_sum(sum);
