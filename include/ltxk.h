@@ -376,6 +376,20 @@ int ltxk_attention(void *out, const void *q, int64_t q_bstride, int64_t q_tstrid
                    int64_t batch, int64_t tokens_q, int64_t tokens_k, int64_t heads, int64_t head_dim, float scale,
                    void *workspace, int64_t workspace_bytes, void *stream);
 
+/* Bytes of workspace ltxk_linear needs for this shape (at most 64 MB). */
+int64_t ltxk_linear_workspace_bytes(int64_t m, int64_t n, int64_t k);
+
+/* y = round(x w^T + bias) for bf16 x [m, k], w [n, k], y [m, n], bias [n] or NULL,
+ * all contiguous and 16-byte aligned; fp32 sums, bias added in fp32, one
+ * rounding.  n is a multiple of 8, k of 64; x, w and y hold at most 2^31
+ * elements each.  Output tiles past the last full wave of the chip are cut over
+ * k, their fp32 sums held in `workspace` (ltxk_linear_workspace_bytes, 16-byte
+ * aligned; NULL if that is 0).  For the projections that a library product
+ * leaves to few compute units: the feature extractor's (k = 188160,
+ * standalone/ltx_te.py:179-184) and the FFN's second one (ltx_nn.py:247-248). */
+int ltxk_linear(void *y, const void *x, const void *w, const void *bias, int64_t m, int64_t n, int64_t k,
+                void *workspace, int64_t workspace_bytes, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -4,10 +4,10 @@
 Kept as in the reference (names, signatures, shapes): rms_norm, sdpa,
 generate_freq_grid_np/_pytorch, precompute_freqs_cis, apply_split_rotary_emb,
 TimestepEmbedder, CombinedTimestepEmbeddings, AdaLayerNormSingle, Attention,
-FeedForward.  Linear layers stay on PyTorch-ROCm; RMSNorm, q/k norm + split
-RoPE, unmasked attention with the per-head gate and GELU-tanh are ltxk kernels,
-with fp32 arithmetic and one bf16 rounding per output.  `sdpa` and masked
-attention are PyTorch-ROCm's.
+FeedForward.  RMSNorm, q/k norm + split RoPE, unmasked attention with the
+per-head gate, GELU-tanh and the linear layers of long K that `long_k_tiles`
+names are ltxk kernels, with fp32 arithmetic and one bf16 rounding per output.
+The other linear layers, `sdpa` and masked attention are PyTorch-ROCm's.
 """
 
 import functools
@@ -375,6 +375,37 @@ class Attention(torch.nn.Module):
         return self.to_out(out)
 
 
+def long_k_tiles(m: int, n: int, k: int) -> bool:
+    """Whether a product of (m, k) and (n, k) matrices goes to ltxk_linear: the
+    shapes that leave the library's product to few compute units for a long K
+    (256 x 256 output tiles, 256 at a time).  Measured, library / ltxk_linear, us:
+      K 188160 x N 4096 (2048), M 128: 586 / 371 (404 / 192), 512: 1048 / 673
+        (742 / 363), 1024: 2100 / 1214 (1087 / 632);
+      K 16384 x N 4096, up to 64 tiles, M 256: 50 / 50, 512: 86 / 73, 1024: 124 / 121
+        (80 tiles and more: no faster, M 2048: 207 / 226);
+      the same with 1 to 32 tiles past a full wave, M 4160: 841 / 439, 4608: 907 /
+        486, 8580: 1274 / 901 (48 tiles, M 4800: 507 / 504; 128, M 6144: 601 / 621);
+      K 8192 and less: the library's is faster (M 1008, N 2048: 46 / 49)."""
+    if n % 8 or k % 64 or k < 16384 or max(m * k, n * k, m * n) >= 2**31:
+        return False
+    tiles = -(-m // 256) * -(-n // 256)
+    return k >= 65536 or tiles <= 64 or (tiles > 256 and 0 < tiles % 256 <= 32)
+
+
+def linear(layer: torch.nn.Linear, x: torch.Tensor) -> torch.Tensor:
+    """layer(x), on ltxk_linear where long_k_tiles says so and the call is a plain
+    bf16 product: no hooks, no gradient to record, no autocast."""
+    w, b = layer.weight, layer.bias
+    if (type(layer) is torch.nn.Linear and x.is_cuda and x.shape[-1] == w.shape[1] and x.numel()
+            and long_k_tiles(x.numel() // x.shape[-1], w.shape[0], w.shape[1])
+            and not (layer._forward_hooks or layer._forward_pre_hooks or torch.is_autocast_enabled("cuda"))
+            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or (b is not None and b.requires_grad)))
+            and all(t is None or (t.device == x.device and t.dtype == torch.bfloat16 and t.is_contiguous()
+                                  and t.data_ptr() % 16 == 0) for t in (x, w, b))):
+        return ltxk.linear(x, w, b)
+    return layer(x)
+
+
 class FeedForward(torch.nn.Module):
     """proj_in -> GELU-tanh (ltxk, in place) -> proj_out (ltx_nn.py:239-248)."""
 
@@ -388,4 +419,4 @@ class FeedForward(torch.nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         hdn = self.proj_in(x)
         ltxk.gelu_tanh(hdn, out=hdn)
-        return self.proj_out(hdn)
+        return linear(self.proj_out, hdn)

@@ -25,7 +25,7 @@ import torch
 
 import ltxk
 from common import DEVICE, load_state_dict, read_metadata
-from ltx_nn import Attention, FeedForward, precompute_freqs_cis
+from ltx_nn import Attention, FeedForward, linear, precompute_freqs_cis
 
 
 class FeatureExtractorV2(torch.nn.Module):
@@ -46,7 +46,7 @@ class FeatureExtractorV2(torch.nn.Module):
         layers = [h.contiguous() for h in hidden_states]
         v_in, a_in = ltxk.feature_norm(layers, attention_mask, math.sqrt(vd / self.embedding_dim),
                                        math.sqrt(ad / self.embedding_dim), eps=1e-6)
-        return self.video_aggregate_embed(v_in), self.audio_aggregate_embed(a_in)
+        return linear(self.video_aggregate_embed, v_in), linear(self.audio_aggregate_embed, a_in)
 
 
 class ConnectorBlock(torch.nn.Module):

@@ -119,6 +119,8 @@ SIGNATURES = {
         [_c_vp, _c_vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_vp, _c_i64, _c_i64,
          _c_i64, _c_i64, _c_i64, _c_vp],
     ),
+    "ltxk_linear_workspace_bytes": (_c_i64, [_c_i64] * 3),
+    "ltxk_linear": (_c_int, [_c_vp, _c_vp, _c_vp, _c_vp, _c_i64, _c_i64, _c_i64, _c_vp, _c_i64, _c_vp]),
     "ltxk_attention_workspace_bytes": (_c_i64, [_c_i64] * 5),
     "ltxk_attention": (
         _c_int,
@@ -781,6 +783,27 @@ def attn_combine(part: torch.Tensor, lse: torch.Tensor, parts: int, logits: torc
     rc = load().ltxk_attn_combine(_ptr(out), _ptr(part), parts * ps[0], ps[0], ps[1], ps[2], _ptr(lse),
                                   parts * ls[0], ls[0], ls[1], ls[2], _ptr(logits), b, parts, t, h, dh, _stream(part))
     _check_rc(rc, "attn_combine")
+    return out
+
+
+def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
+    """x (..., K) weight (N, K)^T + bias (N) on the matrix cores; N a multiple of 8, K of 64."""
+    _dev(x, "x")
+    _dev(weight, "weight")
+    n, k = weight.shape
+    if x.shape[-1] != k:
+        raise ValueError(f"x {tuple(x.shape)} does not end in the weight's {k} columns")
+    if bias is not None:
+        _dev(bias, "bias")
+        if bias.numel() != n:
+            raise ValueError(f"bias has {bias.numel()} entries, expected {n}")
+    m = x.numel() // k
+    out = torch.empty(*x.shape[:-1], n, device=x.device, dtype=x.dtype)
+    lib = load()
+    nbytes = lib.ltxk_linear_workspace_bytes(m, n, k)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device) if nbytes else None
+    rc = lib.ltxk_linear(_ptr(out), x.data_ptr(), weight.data_ptr(), _ptr(bias), m, n, k, _ptr(ws), nbytes, _stream(x))
+    _check_rc(rc, "linear")
     return out
 
 

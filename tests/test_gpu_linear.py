@@ -1,0 +1,80 @@
+"""ltxk_linear (csrc/gemm.hip) against the product in fp64, and the layers that
+take it against torch's own linear (GPU)."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda")
+
+
+def _case(m, n, k, bias, seed=0):
+    g = torch.Generator(device=DEV).manual_seed(m + n + k + seed)
+    x = torch.randn(m, k, device=DEV, generator=g).to(torch.bfloat16)
+    w = (torch.randn(n, k, device=DEV, generator=g) * 0.05).to(torch.bfloat16)
+    b = torch.randn(n, device=DEV, generator=g).to(torch.bfloat16) if bias else None
+    return x, w, b
+
+
+def _check(x, w, b, got):
+    """fp32 sums of k exact products move by at most k 2^-24 of the sum of their
+    sizes (in any order), the rounding to bf16 by 2^-8 of the result."""
+    k = x.shape[-1]
+    for r in range(0, x.shape[0], 512):
+        xr = x[r:r + 512].double()
+        want, size = xr @ w.double().T, xr.abs() @ w.double().abs().T
+        if b is not None:
+            want, size = want + b.double(), size + b.double().abs()
+        err = (got[r:r + 512].double() - want).abs()
+        assert bool((err <= want.abs() * 2.0**-8 + size * k * 2.0**-24 + 1e-30).all()), f"rows {r}.."
+
+
+@pytest.mark.parametrize("m,n,k,bias", [
+    (1, 8, 64, True), (1, 256, 128, False), (255, 264, 192, True), (257, 256, 64 * 9, True), (300, 520, 4096, False),
+    (129, 2048, 8192, True), (1000, 1024, 16448, True),
+    (4100, 4096, 128, True), (4352, 4096, 1088, False), (4097, 4104, 320, True)])
+def test_linear_matches_fp64(m, n, k, bias):
+    """One tile and its edges, tiles cut over K, and a full wave of tiles with
+    some past it."""
+    import ltxk
+
+    x, w, b = _case(m, n, k, bias)
+    _check(x, w, b, ltxk.linear(x, w, b))
+
+
+def test_refusals():
+    import ltxk
+
+    lib = ltxk.load()
+    x, w, _ = _case(16, 64, 128, False)
+    y = torch.empty(16, 64, device=DEV, dtype=torch.bfloat16)
+
+    def call(n=64, k=128, ws=0, shift=0):
+        return lib.ltxk_linear(y.data_ptr(), x.data_ptr() + shift, w.data_ptr(), None, 16, n, k, None, ws, None)
+
+    assert call(n=60) == ltxk.E_ARG and call(k=96) == ltxk.E_ARG and call(shift=2) == ltxk.E_ALIGN
+    assert lib.ltxk_linear_workspace_bytes(16, 64, 128) > 0 and call() == ltxk.E_ARG  # no workspace
+    with pytest.raises(ValueError):
+        ltxk.linear(x, w[:, :64].contiguous())
+
+
+@pytest.mark.parametrize("shape,n,bias,own", [((1, 300), 256, True, True), ((2, 33), 264, False, True),
+                                              ((7,), 512, True, True), ((5,), 500, True, False)])
+def test_layer_route(shape, n, bias, own):
+    """ltx_nn.linear on torch.nn.Linear of K 16384: its route by shape, by hook and
+    by recorded gradient, and its values against the layer's own."""
+    import ltx_nn
+
+    layer = torch.nn.Linear(16384, n, bias=bias, device=DEV, dtype=torch.bfloat16)
+    x = torch.randn(*shape, 16384, device=DEV).to(torch.bfloat16)
+    m = x.numel() // 16384
+    assert ltx_nn.long_k_tiles(m, n, 16384) == own
+    with torch.no_grad():
+        got, want = ltx_nn.linear(layer, x), layer(x)
+        assert got.shape == want.shape
+        _check(x.reshape(m, -1), layer.weight, layer.bias, got.reshape(m, n))
+        seen = []
+        handle = layer.register_forward_hook(lambda *a: seen.append(1))
+        assert torch.equal(ltx_nn.linear(layer, x), want) and seen == [1]
+        handle.remove()
+    assert ltx_nn.linear(layer, x).requires_grad  # a recorded gradient keeps the layer's own call
