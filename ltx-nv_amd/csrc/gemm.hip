@@ -71,7 +71,7 @@ __device__ __forceinline__ void step_barrier(bool more)
 {
     asm volatile("" ::: "memory");
     if (more)
-        __builtin_amdgcn_s_waitcnt(0x0070 | N);  // vmcnt(N) lgkmcnt(0)
+        __builtin_amdgcn_s_waitcnt(0x0070 | (N & 15) | (N >> 4 << 14));  // vmcnt(N) lgkmcnt(0)
     else
         __builtin_amdgcn_s_waitcnt(0x0070);
     __builtin_amdgcn_s_barrier();
@@ -253,6 +253,116 @@ GemmCut cut(int64_t m, int64_t n, int64_t k)
     return c;
 }
 
+// ------------------------------------------------- several layers, few rows --
+// y_g = round_bf16(x w_g^T + bias_g) for up to four weights over the same few rows
+// of x (an audio stream's q, k, v and gate projections) in one launch.  Layer by
+// layer they take a launch and about 20 us of the host each: [126, 2048] x (3 x 2048
+// + 32) 45 us on the device and 77 in eager calls, here 16 and 16.  What bounds it
+// is each workgroup's own loads (65 of the 95 KB a us that loads alone reach), of
+// which x is most: 128 rows of x and 32 of a weight a workgroup, so that 193 compute
+// units work without a second pass.  Steps of 128 of K: 17 us with 64.
+constexpr int kFewRows = 128, kFewCols = 32, kFewWaves = 4, kMaxLayers = 4;
+constexpr int kFewStep = 2 * kStep;    // elements of K a step, as two tiles of kStep
+constexpr int kFewX = 3, kFewW = 7;    // steps of x and of w in LDS
+
+struct FewLayer {
+    const uint16_t *w, *bias;
+    uint16_t *y;
+    int n, first;  // rows of w; its first column tile
+};
+
+struct FewParams {
+    const uint16_t *x;
+    FewLayer g[kMaxLayers];
+    int m, k, tiles_m, tiles_n;
+};
+
+// Four waves load x and take 32 of its rows each; a fifth only loads w, whose
+// rows come from memory: a wave's loads return in order, so beside x, which the L2
+// holds, they could not run as far ahead.
+__global__ void __launch_bounds__((kFewWaves + 1) * 64, 1) few_rows_kernel(FewParams p)
+{
+    constexpr int kXBytes = kFewRows * kFewStep * 2, kWBytes = kFewCols * kFewStep * 2, L = 8;  // loads of a wave a step
+    __shared__ __attribute__((aligned(1024))) char smem[kFewX * kXBytes + kFewW * kWBytes];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int l32 = lane & 31, half = lane >> 5;
+
+    // a weight's tile goes to one XCD for all tiles of x
+    const int t = (blockIdx.x >> 3) / p.tiles_m * 8 + (blockIdx.x & 7), m0 = (blockIdx.x >> 3) % p.tiles_m * kFewRows;
+    if (t >= p.tiles_n) return;
+    FewLayer g = p.g[0];
+#pragma unroll
+    for (int i = 1; i < kMaxLayers; ++i)
+        if (t >= p.g[i].first) g = p.g[i];
+    const int n0 = (t - g.first) * kFewCols, n = p.k / kFewStep;
+
+    // rows past the last repeat it; their results are not stored
+    const bool is_x = wave < kFewWaves;
+    const uint64_t base = reinterpret_cast<uint64_t>(is_x ? p.x : g.w);
+    const u32x4 rsrc = {static_cast<uint32_t>(base), static_cast<uint32_t>(base >> 32) & 0xffff, 0xffffffffu, 0x00020000u};
+    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_char *)smem)) +
+                          (is_x ? wave * 4096 : kFewX * kXBytes);
+    uint32_t go[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int row = ((is_x ? wave : 0) * 4 + j) * 8 + (lane >> 3);
+        const int at = is_x ? min(m0 + row, p.m - 1) : min(n0 + row, g.n - 1);
+        go[j] = static_cast<uint32_t>(at) * (static_cast<uint32_t>(p.k) * 2) + chunk_pos(row, lane & 7) * 16;
+    }
+    auto load = [&](int i, int slot) {
+#pragma unroll
+        for (int j = 0; j < L; ++j)
+            load_lds(rsrc,
+                     __builtin_amdgcn_readfirstlane(lds0 + slot + (j >> 2) * ((is_x ? kFewRows : kFewCols) * kStep * 2) +
+                                                    (j & 3) * 1024),
+                     go[j & 3], __builtin_amdgcn_readfirstlane((2 * i + (j >> 2)) * kStep * 2));
+    };
+    // At barrier i step i is there and step i - 1 read by all: its slot takes the
+    // load that is furthest ahead.
+    if (!is_x) {
+        for (int i = 0; i < kFewW - 1 && i < n; ++i) load(i, i * kWBytes);
+        for (int i = 0; i < n; ++i) {
+            step_barrier<(kFewW - 2) * L>(i + kFewW - 2 < n);
+            if (i + kFewW - 1 < n) load(i + kFewW - 1, (i + kFewW - 1) % kFewW * kWBytes);
+        }
+        return;
+    }
+    for (int i = 0; i < kFewX - 1 && i < n; ++i) load(i, i * kXBytes);
+
+    int off[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) off[s] = l32 * 128 + chunk_pos(l32, 2 * s + half) * 16;
+    f32x16 acc2[2] = {};
+    for (int i = 0; i < n; ++i) {
+        step_barrier<(kFewX - 2) * L>(i + kFewX - 2 < n);
+        const char *xs = smem + i % kFewX * kXBytes + wave * 4096, *ws = smem + kFewX * kXBytes + i % kFewW * kWBytes;
+        bf16x8 xf[8], wf[8];
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            xf[s] = *reinterpret_cast<const bf16x8 *>(xs + (s >> 2) * (kFewRows * kStep * 2) + off[s & 3]);
+            wf[s] = *reinterpret_cast<const bf16x8 *>(ws + (s >> 2) * (kFewCols * kStep * 2) + off[s & 3]);
+        }
+        if (i + kFewX - 1 < n) load(i + kFewX - 1, (i + kFewX - 1) % kFewX * kXBytes);
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+            acc2[s & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[s], xf[s], acc2[s & 1], 0, 0, 0);
+    }
+    const f32x16 acc = acc2[0] + acc2[1];
+
+    const int row = m0 + wave * 32 + l32;
+    if (row >= p.m) return;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int col = n0 + 8 * q + 4 * half;
+        if (col >= g.n) continue;
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = acc[4 * q + e] + (g.bias ? bf16_to_f32(g.bias[col + e]) : 0.f);
+        *reinterpret_cast<uint2 *>(g.y + static_cast<int64_t>(row) * g.n + col) =
+            make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+    }
+}
+
 }  // namespace
 }  // namespace ltxk
 
@@ -303,5 +413,54 @@ extern "C" int ltxk_linear(void *y, const void *x, const void *w, const void *bi
     const unsigned grid = 8u * static_cast<unsigned>(c.whole / 8 + (c.rest * c.parts + 7) / 8);
     gemm_kernel<<<grid, kWaves * 64, 0, s>>>(p);
     if (c.rest) gemm_sum_kernel<<<static_cast<unsigned>(c.rest) * (kTile * kTile / 8 / 256), 256, 0, s>>>(p);
+    return check_launch(what);
+}
+
+extern "C" int ltxk_linear_layers(void *const *y, const void *x, const void *const *w, const void *const *bias,
+                                  const int64_t *n, int64_t layers, int64_t m, int64_t k, void *stream)
+{
+    static const char *what = "linear_layers";
+    clear_error();
+    if (layers < 1 || layers > kMaxLayers)
+        return fail(LTXK_E_ARG, "%s: 1 to %d layers (got %lld)", what, kMaxLayers, (long long)layers);
+    if (m < 0 || k <= 0 || k % kFewStep)
+        return fail(LTXK_E_ARG, "%s: bad shape m=%lld k=%lld (k a multiple of %d)", what, (long long)m, (long long)k,
+                    kFewStep);
+    if (!y || !w || !n) return fail(LTXK_E_ARG, "%s: null y, w or n", what);
+    if (m == 0) return LTXK_OK;
+    const int64_t kMax = int64_t{1} << 31;
+    if (!x) return fail(LTXK_E_ARG, "%s: null x", what);
+    if (!aligned16(x)) return fail(LTXK_E_ALIGN, "%s: x must be 16-byte aligned", what);
+    if (k >= kMax / 2 || m > kMax / k) return fail(LTXK_E_ARG, "%s: x spans 2^32 bytes or more", what);
+    FewParams p{};
+    p.x = static_cast<const uint16_t *>(x);
+    p.m = static_cast<int>(m);
+    p.k = static_cast<int>(k);
+    p.tiles_m = static_cast<int>((m + kFewRows - 1) / kFewRows);
+    int64_t tiles = 0;
+    for (int64_t i = 0; i < kMaxLayers; ++i) {
+        FewLayer &g = p.g[i];
+        if (i >= layers) {
+            g.first = 0x7fffffff;  // no tile reaches it
+            continue;
+        }
+        const void *b = bias ? bias[i] : nullptr;
+        if (n[i] <= 0 || n[i] % 8 || n[i] > kMax / k || m > kMax / n[i])
+            return fail(LTXK_E_ARG, "%s: layer %lld: n must be a positive multiple of 8 within 2^31 elements (got %lld)",
+                        what, (long long)i, (long long)n[i]);
+        if (!y[i] || !w[i]) return fail(LTXK_E_ARG, "%s: layer %lld: null y or w", what, (long long)i);
+        if (!aligned16(y[i]) || !aligned16(w[i]) || !aligned16(b))
+            return fail(LTXK_E_ALIGN, "%s: layer %lld: y, w and bias must be 16-byte aligned", what, (long long)i);
+        g.w = static_cast<const uint16_t *>(w[i]);
+        g.bias = static_cast<const uint16_t *>(b);
+        g.y = static_cast<uint16_t *>(y[i]);
+        g.n = static_cast<int>(n[i]);
+        g.first = static_cast<int>(tiles);
+        tiles += (n[i] + kFewCols - 1) / kFewCols;
+    }
+    p.tiles_n = static_cast<int>(tiles);
+    const int64_t grid = 8 * ((tiles + 7) / 8) * p.tiles_m;
+    if (grid >= kMax) return fail(LTXK_E_ARG, "%s: too many tiles", what);
+    few_rows_kernel<<<static_cast<unsigned>(grid), (kFewWaves + 1) * 64, 0, static_cast<hipStream_t>(stream)>>>(p);
     return check_launch(what);
 }

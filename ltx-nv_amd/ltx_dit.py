@@ -34,7 +34,8 @@ import torch
 
 import ltxk
 from common import DEVICE, load_state_dict, read_metadata
-from ltx_nn import AdaLayerNormSingle, Attention, FeedForward, precompute_freqs_cis, precompute_freqs_cis_compact
+from ltx_nn import (AdaLayerNormSingle, Attention, FeedForward, precompute_freqs_cis, precompute_freqs_cis_compact,
+                    project)
 from torch_rng import TorchRNG
 
 # ---------------------------------------------------------------------------
@@ -582,10 +583,9 @@ class Block(torch.nn.Module):
         # keys share the video time-axis tables and rotate in one launch
         q_a2v = g_a2v = k_v2a = v_v2a = None
         if do_a2v:
-            q_a2v = A.to_q(a2v_v)
-            g_a2v = A.to_gate_logits(a2v_v).contiguous() if A.to_gate_logits is not None else None
+            q_a2v, g_a2v = project(a2v_v, A.to_q, A.to_gate_logits)
         if do_v2a:
-            k_v2a, v_v2a = V.to_k(v2a_v), V.to_v(v2a_v)
+            k_v2a, v_v2a = project(v2a_v, V.to_k, V.to_v)
         _qk_pair(A, V, q_a2v, k_v2a, video.cross_pe)
         main_ready, side_ready = ev["main_ready"], ev["side_ready"]
         main_ready.record(main)
@@ -597,10 +597,9 @@ class Block(torch.nn.Module):
             ax, a2v_a, v2a_a = res[0], res[1] if do_a2v else None, res[-1] if do_v2a else None
             q_v2a = g_v2a = None
             if do_a2v:
-                k_a2v, v_a2v = A.to_k(a2v_a), A.to_v(a2v_a)
+                k_a2v, v_a2v = project(a2v_a, A.to_k, A.to_v)
             if do_v2a:
-                q_v2a = V.to_q(v2a_a)
-                g_v2a = V.to_gate_logits(v2a_a).contiguous() if V.to_gate_logits is not None else None
+                q_v2a, g_v2a = project(v2a_a, V.to_q, V.to_gate_logits)
             _qk_pair(A, V, k_a2v, q_v2a, audio.cross_pe, k_first=True)
             side_ready.record(side)
             if do_v2a:

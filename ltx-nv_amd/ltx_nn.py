@@ -5,9 +5,10 @@ Kept as in the reference (names, signatures, shapes): rms_norm, sdpa,
 generate_freq_grid_np/_pytorch, precompute_freqs_cis, apply_split_rotary_emb,
 TimestepEmbedder, CombinedTimestepEmbeddings, AdaLayerNormSingle, Attention,
 FeedForward.  RMSNorm, q/k norm + split RoPE, unmasked attention with the
-per-head gate, GELU-tanh and the linear layers of long K that `long_k_tiles`
-names are ltxk kernels, with fp32 arithmetic and one bf16 rounding per output.
-The other linear layers, `sdpa` and masked attention are PyTorch-ROCm's.
+per-head gate, GELU-tanh, the linear layers of long K that `long_k_tiles` names
+and the projections of few rows (`project`) are ltxk kernels, with fp32
+arithmetic and one bf16 rounding per output.  The other linear layers, `sdpa` and
+masked attention are PyTorch-ROCm's.
 """
 
 import functools
@@ -286,6 +287,69 @@ class AdaLayerNormSingle(torch.nn.Module):
 
 
 # ---------------------------------------------------------------------------
+# Linear layers
+# ---------------------------------------------------------------------------
+
+
+def long_k_tiles(m: int, n: int, k: int) -> bool:
+    """Whether a product of (m, k) and (n, k) matrices goes to ltxk_linear: the
+    shapes that leave the library's product to few compute units for a long K
+    (256 x 256 output tiles, 256 at a time).  Measured, library / ltxk_linear, us:
+      K 188160 x N 4096 (2048), M 128: 586 / 371 (404 / 192), 512: 1048 / 673
+        (742 / 363), 1024: 2100 / 1214 (1087 / 632);
+      K 16384 x N 4096, up to 64 tiles, M 256: 50 / 50, 512: 86 / 73, 1024: 124 / 121
+        (80 tiles and more: no faster, M 2048: 207 / 226);
+      the same with 1 to 32 tiles past a full wave, M 4160: 841 / 439, 4608: 907 /
+        486, 8580: 1274 / 901 (48 tiles, M 4800: 507 / 504; 128, M 6144: 601 / 621);
+      K 8192 and less: the library's is faster (M 1008, N 2048: 46 / 49)."""
+    if n % 8 or k % 64 or k < 16384 or max(m * k, n * k, m * n) >= 2**31:
+        return False
+    tiles = -(-m // 256) * -(-n // 256)
+    return k >= 65536 or tiles <= 64 or (tiles > 256 and 0 < tiles % 256 <= 32)
+
+
+def _plain(layer: torch.nn.Linear, x: torch.Tensor) -> bool:
+    """Whether layer(x) is a bf16 product that the ltxk kernels can take over: a
+    bare torch.nn.Linear without hooks, contiguous aligned operands on x's device,
+    no autocast and no gradient to record."""
+    if type(layer) is not torch.nn.Linear or layer._forward_hooks or layer._forward_pre_hooks:
+        return False
+    w, b = layer.weight, layer.bias
+    if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or (b is not None and b.requires_grad)):
+        return False
+    return x.is_cuda and x.numel() > 0 and x.shape[-1] == w.shape[1] and not torch.is_autocast_enabled("cuda") and all(
+        t is None or (t.device == x.device and t.dtype == torch.bfloat16 and t.is_contiguous() and t.data_ptr() % 16 == 0)
+        for t in (x, w, b))
+
+
+def linear(layer: torch.nn.Linear, x: torch.Tensor) -> torch.Tensor:
+    """layer(x), on ltxk_linear where long_k_tiles says so."""
+    if type(layer) is torch.nn.Linear and long_k_tiles(x.numel() // max(x.shape[-1], 1), *layer.weight.shape) \
+            and _plain(layer, x):
+        return ltxk.linear(x, layer.weight, layer.bias)
+    return layer(x)
+
+
+# ltxk_linear_layers takes the projections of an input of at most this many
+# elements: a launch and about 20 us of the host for all of them instead of for
+# each.  Measured, layer by layer / ltxk_linear_layers, device us (eager calls):
+#   x [126, 2048], N 3 x 2048 + 32: 45 / 16 (77 / 16); [252, 2048]: 47 / 27;
+#   [504, 2048]: 49 / 50; x [126, 4096], N 3 x 4096 + 32: 62 / 50; [256, 4096]: 79 / 87;
+#   one layer alone, x [126, 2048], N 2048: 9 / 13, so single layers stay as they are.
+FEW_ROWS_MAX = 1 << 19
+
+
+def project(x: torch.Tensor, *layers: torch.nn.Linear | None) -> list:
+    """[layer(x) for each layer], None for None, in one launch where x is small."""
+    real = [layer for layer in layers if layer is not None]
+    if 2 <= len(real) <= ltxk.MAX_LINEAR_LAYERS and x.numel() <= FEW_ROWS_MAX and x.shape[-1] % 128 == 0 \
+            and all(_plain(layer, x) and layer.weight.shape[0] % 8 == 0 for layer in real):
+        done = iter(ltxk.linear_layers(x, [layer.weight for layer in real], [layer.bias for layer in real]))
+        return [None if layer is None else next(done) for layer in layers]
+    return [None if layer is None else linear(layer, x) for layer in layers]
+
+
+# ---------------------------------------------------------------------------
 # Attention + FFN
 # ---------------------------------------------------------------------------
 
@@ -293,10 +357,10 @@ class AdaLayerNormSingle(torch.nn.Module):
 class Attention(torch.nn.Module):
     """Multi-head attention with RMS q/k-norm, split RoPE and per-head gating (ltx_nn.py:166-236).
 
-    q/k/v projections are PyTorch-ROCm.  q_norm/k_norm + RoPE run as one
-    in-place ltxk_qk_norm_rope launch on the fresh projections; attention, the
-    head merge and the per-head 2*sigmoid gate are one ltxk_attention call
-    (`attend`).
+    q/k/v/gate projections are PyTorch-ROCm, or one ltxk_linear_layers launch
+    over few rows (`project`).  q_norm/k_norm + RoPE run as one in-place
+    ltxk_qk_norm_rope launch on the fresh projections; attention, the head merge
+    and the per-head 2*sigmoid gate are one ltxk_attention call (`attend`).
     """
 
     def __init__(self, query_dim: int, context_dim: int | None = None, heads: int = 8, dim_head: int = 64,
@@ -319,15 +383,18 @@ class Attention(torch.nn.Module):
                 k_pe: tuple[torch.Tensor, torch.Tensor] | None = None,
                 perturbation_mask: torch.Tensor | None = None, all_perturbed: bool = False) -> torch.Tensor:
         context = x if context is None else context
-        b = x.shape[0]
         h, dh = self.heads, self.dim_head
-        v = self.to_v(context)
-        gates = self.to_gate_logits(x).contiguous() if self.to_gate_logits is not None else None
         if all_perturbed:
+            v = self.to_v(context)
+            gates = self.to_gate_logits(x).contiguous() if self.to_gate_logits is not None else None
             out = v if gates is None else ltxk.head_gate(v, gates)
             return self.to_out(out)
-        q = self.to_q(x)
-        k = self.to_k(context)
+        if context is x:
+            q, k, v, gates = project(x, self.to_q, self.to_k, self.to_v, self.to_gate_logits)
+        else:
+            q, gates = project(x, self.to_q, self.to_gate_logits)
+            k, v = project(context, self.to_k, self.to_v)
+        gates = gates.contiguous() if gates is not None else None
         ltxk.qk_norm_rope(q, k, h, dh, q_weight=self.q_norm.weight, k_weight=self.k_norm.weight,
                           q_pe=pe, k_pe=pe if k_pe is None else k_pe, eps=self.eps)
         return self.attend(q, k, v, gates, mask, perturbation_mask)
@@ -373,37 +440,6 @@ class Attention(torch.nn.Module):
             # head merge [+ perturbation blend] [+ per-head gate] in one pass
             out = ltxk.head_gate(attn, gates, v=v.contiguous() if pm is not None else None, mask=pm)
         return self.to_out(out)
-
-
-def long_k_tiles(m: int, n: int, k: int) -> bool:
-    """Whether a product of (m, k) and (n, k) matrices goes to ltxk_linear: the
-    shapes that leave the library's product to few compute units for a long K
-    (256 x 256 output tiles, 256 at a time).  Measured, library / ltxk_linear, us:
-      K 188160 x N 4096 (2048), M 128: 586 / 371 (404 / 192), 512: 1048 / 673
-        (742 / 363), 1024: 2100 / 1214 (1087 / 632);
-      K 16384 x N 4096, up to 64 tiles, M 256: 50 / 50, 512: 86 / 73, 1024: 124 / 121
-        (80 tiles and more: no faster, M 2048: 207 / 226);
-      the same with 1 to 32 tiles past a full wave, M 4160: 841 / 439, 4608: 907 /
-        486, 8580: 1274 / 901 (48 tiles, M 4800: 507 / 504; 128, M 6144: 601 / 621);
-      K 8192 and less: the library's is faster (M 1008, N 2048: 46 / 49)."""
-    if n % 8 or k % 64 or k < 16384 or max(m * k, n * k, m * n) >= 2**31:
-        return False
-    tiles = -(-m // 256) * -(-n // 256)
-    return k >= 65536 or tiles <= 64 or (tiles > 256 and 0 < tiles % 256 <= 32)
-
-
-def linear(layer: torch.nn.Linear, x: torch.Tensor) -> torch.Tensor:
-    """layer(x), on ltxk_linear where long_k_tiles says so and the call is a plain
-    bf16 product: no hooks, no gradient to record, no autocast."""
-    w, b = layer.weight, layer.bias
-    if (type(layer) is torch.nn.Linear and x.is_cuda and x.shape[-1] == w.shape[1] and x.numel()
-            and long_k_tiles(x.numel() // x.shape[-1], w.shape[0], w.shape[1])
-            and not (layer._forward_hooks or layer._forward_pre_hooks or torch.is_autocast_enabled("cuda"))
-            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or (b is not None and b.requires_grad)))
-            and all(t is None or (t.device == x.device and t.dtype == torch.bfloat16 and t.is_contiguous()
-                                  and t.data_ptr() % 16 == 0) for t in (x, w, b))):
-        return ltxk.linear(x, w, b)
-    return layer(x)
 
 
 class FeedForward(torch.nn.Module):

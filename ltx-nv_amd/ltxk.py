@@ -121,6 +121,11 @@ SIGNATURES = {
     ),
     "ltxk_linear_workspace_bytes": (_c_i64, [_c_i64] * 3),
     "ltxk_linear": (_c_int, [_c_vp, _c_vp, _c_vp, _c_vp, _c_i64, _c_i64, _c_i64, _c_vp, _c_i64, _c_vp]),
+    "ltxk_linear_layers": (
+        _c_int,
+        [ctypes.POINTER(_c_vp), _c_vp, ctypes.POINTER(_c_vp), ctypes.POINTER(_c_vp), ctypes.POINTER(_c_i64), _c_i64,
+         _c_i64, _c_i64, _c_vp],
+    ),
     "ltxk_attention_workspace_bytes": (_c_i64, [_c_i64] * 5),
     "ltxk_attention": (
         _c_int,
@@ -805,6 +810,34 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
     rc = lib.ltxk_linear(_ptr(out), x.data_ptr(), weight.data_ptr(), _ptr(bias), m, n, k, _ptr(ws), nbytes, _stream(x))
     _check_rc(rc, "linear")
     return out
+
+
+MAX_LINEAR_LAYERS = 4
+
+
+def linear_layers(x: torch.Tensor, weights, biases) -> list[torch.Tensor]:
+    """[x weight^T + bias] for up to four layers over the same few rows x (..., K) in
+    one launch; weights (N_i, K) with N_i a multiple of 8, K of 128; a bias may be None."""
+    _dev(x, "x")
+    k, count = x.shape[-1], len(weights)
+    if not 1 <= count <= MAX_LINEAR_LAYERS or len(biases) != count:
+        raise ValueError(f"1 to {MAX_LINEAR_LAYERS} weights with a bias (or None) each")
+    outs = []
+    for w, b in zip(weights, biases):
+        _dev(w, "weight")
+        if w.ndim != 2 or w.shape[1] != k:
+            raise ValueError(f"weight {tuple(w.shape)} does not take x {tuple(x.shape)}")
+        if b is not None:
+            _dev(b, "bias")
+            if b.numel() != w.shape[0]:
+                raise ValueError(f"bias has {b.numel()} entries, expected {w.shape[0]}")
+        outs.append(torch.empty(*x.shape[:-1], w.shape[0], device=x.device, dtype=x.dtype))
+    ptrs = _c_vp * count
+    rc = load().ltxk_linear_layers(ptrs(*[o.data_ptr() for o in outs]), x.data_ptr(),
+                                   ptrs(*[w.data_ptr() for w in weights]), ptrs(*[_ptr(b) for b in biases]),
+                                   (_c_i64 * count)(*[w.shape[0] for w in weights]), count, x.numel() // k, k, _stream(x))
+    _check_rc(rc, "linear_layers")
+    return outs
 
 
 ATTENTION_HEAD_DIMS = (64, 128)

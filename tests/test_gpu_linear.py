@@ -42,6 +42,38 @@ def test_linear_matches_fp64(m, n, k, bias):
     _check(x, w, b, ltxk.linear(x, w, b))
 
 
+@pytest.mark.parametrize("m,k,ns,biased", [
+    (1, 128, (8,), (True,)), (126, 2048, (2048, 2048, 2048, 32), (True, True, False, True)),
+    (129, 384, (40, 32), (True, True)), (300, 256, (264, 8, 64), (False, True, True)), (128, 896, (72, 96), (True, False)),
+    (33, 4096, (128, 128, 128, 32), (True, True, True, True))])
+def test_layers_over_few_rows(m, k, ns, biased):
+    """One launch for several layers: each equals its product in fp64, over edges
+    of the 128-row and 32-column tiles and K of one step to more than its rings."""
+    import ltxk
+
+    cases = [_case(m, n, k, b, seed=i) for i, (n, b) in enumerate(zip(ns, biased))]
+    x = cases[0][0]
+    outs = ltxk.linear_layers(x, [c[1] for c in cases], [c[2] for c in cases])
+    for (_, w, b), y in zip(cases, outs):
+        _check(x, w, b, y)
+
+
+@pytest.mark.parametrize("rows,own", [(126, True), (257, False)])
+def test_projection_route(rows, own):
+    """ltx_nn.project on rows of 2048: one launch up to 2^19 elements of x, the
+    layers' own calls above, a missing layer as None."""
+    import ltx_nn
+
+    layers = [torch.nn.Linear(2048, n, device=DEV, dtype=torch.bfloat16) for n in (2048, 32)]
+    x = torch.randn(1, rows, 2048, device=DEV).to(torch.bfloat16)
+    assert (x.numel() <= ltx_nn.FEW_ROWS_MAX) == own
+    with torch.no_grad():
+        q, none, g = ltx_nn.project(x, layers[0], None, layers[1])
+    assert none is None and q.shape == (1, rows, 2048) and g.shape == (1, rows, 32)
+    for layer, y in zip(layers, (q, g)):
+        _check(x[0], layer.weight.detach(), layer.bias.detach(), y[0])
+
+
 def test_refusals():
     import ltxk
 
@@ -56,6 +88,12 @@ def test_refusals():
     assert lib.ltxk_linear_workspace_bytes(16, 64, 128) > 0 and call() == ltxk.E_ARG  # no workspace
     with pytest.raises(ValueError):
         ltxk.linear(x, w[:, :64].contiguous())
+    with pytest.raises(ValueError):
+        ltxk.linear_layers(x, [w] * 5, [None] * 5)
+    with pytest.raises(RuntimeError):  # n not a multiple of 8
+        ltxk.linear_layers(x, [w[:12].contiguous(), w], [None, None])
+    with pytest.raises(RuntimeError):  # k not a multiple of 128
+        ltxk.linear_layers(x[:, :64].contiguous(), [w[:, :64].contiguous()], [None])
 
 
 @pytest.mark.parametrize("shape,n,bias,own", [((1, 300), 256, True, True), ((2, 33), 264, False, True),
