@@ -53,15 +53,17 @@ __device__ __forceinline__ void tile_rows(const GemmParams &p, int t, int &m0, i
 // one chunk column, which a fragment read takes at a time, cover all banks.
 __device__ __forceinline__ int chunk_pos(int row, int c) { return c ^ ((row >> 1) & 7); }
 
-// 64 lanes x 16 bytes from memory straight to LDS.  In assembly because the
-// compiler, which cannot tell the buffers of the ring apart, would wait for every
+// 64 lanes x 16 bytes from memory straight to LDS at `lds` (through m0, which the
+// compiler sets anew before any use of its own).  In assembly because the
+// compiler, which cannot tell the buffers of a ring apart, would wait for every
 // load in flight before each LDS read; it has no output register, and its wait is
-// step_barrier's.
+// step_barrier's.  The wait states cover scalar operands that a vector instruction
+// has just written, which the compiler does not see the load read.
 __device__ __forceinline__ void load_lds(const u32x4 &rsrc, uint32_t lds, uint32_t off, uint32_t soff)
 {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                  ::"s"(lds), "v"(off), "s"(rsrc), "s"(soff)
-                 : "memory", "m0");
+                 : "memory");
 }
 
 // At most `N` of this wave's loads in flight (none without `more`) and its LDS
