@@ -18,6 +18,7 @@ import numpy
 import torch
 import torch.nn.functional as F
 from torch.nn.attention import SDPBackend, sdpa_kernel
+from torch.nn.modules.module import _has_any_global_hook
 
 import ltxk
 
@@ -308,25 +309,40 @@ def long_k_tiles(m: int, n: int, k: int) -> bool:
     return k >= 65536 or tiles <= 64 or (tiles > 256 and 0 < tiles % 256 <= 32)
 
 
-def _plain(layer: torch.nn.Linear, x: torch.Tensor) -> bool:
-    """Whether layer(x) is a bf16 product that the ltxk kernels can take over: a
-    bare torch.nn.Linear without hooks, contiguous aligned operands on x's device,
-    no autocast and no gradient to record."""
-    if type(layer) is not torch.nn.Linear or layer._forward_hooks or layer._forward_pre_hooks:
-        return False
-    w, b = layer.weight, layer.bias
-    if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or (b is not None and b.requires_grad)):
-        return False
-    return x.is_cuda and x.numel() > 0 and x.shape[-1] == w.shape[1] and not torch.is_autocast_enabled("cuda") and all(
-        t is None or (t.device == x.device and t.dtype == torch.bfloat16 and t.is_contiguous() and t.data_ptr() % 16 == 0)
-        for t in (x, w, b))
+def _plain_input(x: torch.Tensor) -> bool:
+    """Whether the ltxk products can read x: contiguous aligned bf16 on a ROCm
+    device, no autocast, no gradient to record."""
+    return x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous() and x.data_ptr() % 16 == 0 and x.numel() > 0 \
+        and not (torch.is_grad_enabled() and x.requires_grad) and not torch.is_autocast_enabled("cuda")
+
+
+def _plain_layer(layer: torch.nn.Linear, x: torch.Tensor) -> tuple | None:
+    """(weight, bias) of a bare torch.nn.Linear (no hooks, its own forward, plain
+    tensors) whose operands fit x like _plain_input, else None.  Reads the module's
+    dictionaries: its attribute lookup costs more than the rest (`project` over
+    four layers takes the host 30 us with it, 16 without)."""
+    if type(layer) is not torch.nn.Linear or layer._forward_hooks or layer._forward_pre_hooks \
+            or "forward" in layer.__dict__ or _has_any_global_hook():
+        return None
+    params = layer._parameters
+    w, b = params.get("weight"), params.get("bias")
+    if w is None or w.shape[1] != x.shape[-1]:
+        return None
+    for t in (w, b):
+        if t is not None and not (type(t) in (torch.nn.Parameter, torch.Tensor) and t.get_device() == x.get_device()
+                                  and t.dtype == torch.bfloat16 and t.is_contiguous() and t.data_ptr() % 16 == 0
+                                  and not (t.requires_grad and torch.is_grad_enabled())):
+            return None
+    return w, b
 
 
 def linear(layer: torch.nn.Linear, x: torch.Tensor) -> torch.Tensor:
     """layer(x), on ltxk_linear where long_k_tiles says so."""
-    if type(layer) is torch.nn.Linear and long_k_tiles(x.numel() // max(x.shape[-1], 1), *layer.weight.shape) \
-            and _plain(layer, x):
-        return ltxk.linear(x, layer.weight, layer.bias)
+    if type(layer) is torch.nn.Linear and long_k_tiles(x.numel() // max(x.shape[-1], 1), layer.out_features,
+                                                       x.shape[-1]) and _plain_input(x):
+        plain = _plain_layer(layer, x)
+        if plain is not None:
+            return ltxk.linear(x, *plain)
     return layer(x)
 
 
@@ -343,9 +359,12 @@ def project(x: torch.Tensor, *layers: torch.nn.Linear | None) -> list:
     """[layer(x) for each layer], None for None, in one launch where x is small."""
     real = [layer for layer in layers if layer is not None]
     if 2 <= len(real) <= ltxk.MAX_LINEAR_LAYERS and x.numel() <= FEW_ROWS_MAX and x.shape[-1] % 128 == 0 \
-            and all(_plain(layer, x) and layer.weight.shape[0] % 8 == 0 for layer in real):
-        done = iter(ltxk.linear_layers(x, [layer.weight for layer in real], [layer.bias for layer in real]))
-        return [None if layer is None else next(done) for layer in layers]
+            and _plain_input(x):
+        plain = [_plain_layer(layer, x) for layer in real]
+        if all(p is not None and p[0].shape[0] % 8 == 0 for p in plain):
+            weights, biases = zip(*plain)
+            done = iter(ltxk._launch_layers(x, weights, biases))
+            return [None if layer is None else next(done) for layer in layers]
     return [None if layer is None else linear(layer, x) for layer in layers]
 
 
