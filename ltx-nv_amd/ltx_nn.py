@@ -300,13 +300,29 @@ def long_k_tiles(m: int, n: int, k: int) -> bool:
         (742 / 363), 1024: 2100 / 1214 (1087 / 632);
       K 16384 x N 4096, up to 64 tiles, M 256: 50 / 50, 512: 86 / 73, 1024: 124 / 121
         (80 tiles and more: no faster, M 2048: 207 / 226);
-      the same with 1 to 32 tiles past a full wave, M 4160: 841 / 439, 4608: 907 /
-        486, 8580: 1274 / 901 (48 tiles, M 4800: 507 / 504; 128, M 6144: 601 / 621);
       K 8192 and less: the library's is faster (M 1008, N 2048: 46 / 49)."""
     if n % 8 or k % 64 or k < 16384 or max(m * k, n * k, m * n) >= 2**31:
         return False
-    tiles = -(-m // 256) * -(-n // 256)
-    return k >= 65536 or tiles <= 64 or (tiles > 256 and 0 < tiles % 256 <= 32)
+    return k >= 65536 or -(-m // 256) * -(-n // 256) <= 64
+
+
+def full_wave_rows(m: int, n: int, k: int) -> int:
+    """The rows of a large (m, k) x (n, k) product that fill whole waves of 256 tiles
+    of 256 x 256, where few rows are left past them: those then go in a launch of
+    their own, because the library gives them a whole further wave, or other tiles
+    to all of it.  0: one launch.  Measured, one launch / two, us, N x K:
+      4096 x 4096, M 4160: 142 / 103, 4290: 137 / 107, 4800: 146 / 120, 8580: 221 / 201,
+        17160: 433 / 383;  4096 x 2048, M 4290: 83 / 60, 12500: 230 / 154;
+      16384 x 4096, M 4290: 433 / 383, 4800: 574 / 430, 17160: 1517 / 1524;
+      4096 x 16384, M 4290: 840 / 396, 8448: 1181 / 743, 17160: 1576 / 1525.
+    Above 768 rows the two are less often apart, and once the other way (4096 x 16384,
+    1769 rows past 4096: 584 / 746; 16384 x 4096, 808 past 8192: 790 / 812)."""
+    across = -(-n // 256)
+    if n < 4096 or not 2048 <= k < 65536 or across > 64 or 256 % across:
+        return 0
+    wave = 256 // across * 256
+    main = m // wave * wave
+    return main if main >= 4096 and 0 < m - main <= 768 else 0
 
 
 def _plain_input(x: torch.Tensor) -> bool:
@@ -337,13 +353,32 @@ def _plain_layer(layer: torch.nn.Linear, x: torch.Tensor) -> tuple | None:
 
 
 def linear(layer: torch.nn.Linear, x: torch.Tensor) -> torch.Tensor:
-    """layer(x), on ltxk_linear where long_k_tiles says so."""
-    if type(layer) is torch.nn.Linear and long_k_tiles(x.numel() // max(x.shape[-1], 1), layer.out_features,
-                                                       x.shape[-1]) and _plain_input(x):
+    """layer(x): on ltxk_linear where long_k_tiles says so, in two launches where
+    full_wave_rows does."""
+    if type(layer) is not torch.nn.Linear:
+        return layer(x)
+    k, n = x.shape[-1], layer.out_features
+    m = x.numel() // max(k, 1)
+    own = long_k_tiles(m, n, k)
+    main = 0 if own else full_wave_rows(m, n, k)
+    if (own or main) and _plain_input(x):
         plain = _plain_layer(layer, x)
         if plain is not None:
-            return ltxk.linear(x, *plain)
+            return ltxk.linear(x, *plain) if own else _two_launches(x, *plain, main)
     return layer(x)
+
+
+def _two_launches(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, main: int) -> torch.Tensor:
+    """x weight^T + bias, the first `main` rows and the others apart."""
+    k, n = x.shape[-1], weight.shape[0]
+    out = x.new_empty((*x.shape[:-1], n))
+    rows, to, wt = x.view(-1, k), out.view(-1, n), weight.t()
+    for part in (slice(0, main), slice(main, None)):
+        if bias is None:
+            torch.mm(rows[part], wt, out=to[part])
+        else:
+            torch.addmm(bias, rows[part], wt, out=to[part])
+    return out
 
 
 # ltxk_linear_layers takes the projections of an input of at most this many
@@ -407,7 +442,7 @@ class Attention(torch.nn.Module):
             v = self.to_v(context)
             gates = self.to_gate_logits(x).contiguous() if self.to_gate_logits is not None else None
             out = v if gates is None else ltxk.head_gate(v, gates)
-            return self.to_out(out)
+            return linear(self.to_out, out)
         if context is x:
             q, k, v, gates = project(x, self.to_q, self.to_k, self.to_v, self.to_gate_logits)
         else:
@@ -438,8 +473,8 @@ class Attention(torch.nn.Module):
             pm = perturbation_mask.reshape(-1).to(torch.bfloat16).contiguous()
         if mask is None and fused_attention_applies(q, k, v, h, dh):
             if pm is None:
-                return self.to_out(ltxk.attention(q, k, v, h, gates))
-            return self.to_out(ltxk.head_gate(ltxk.attention(q, k, v, h), gates, v=v, mask=pm, heads=h))
+                return linear(self.to_out, ltxk.attention(q, k, v, h, gates))
+            return linear(self.to_out, ltxk.head_gate(ltxk.attention(q, k, v, h), gates, v=v, mask=pm, heads=h))
         q4 = q.view(b, -1, h, dh).transpose(1, 2)
         k4 = k.view(b, -1, h, dh).transpose(1, 2)
         v4 = v.view(b, -1, h, dh).transpose(1, 2)
@@ -472,6 +507,6 @@ class FeedForward(torch.nn.Module):
         self.proj_out = torch.nn.Linear(inner, dim_out, bias=bias)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        hdn = self.proj_in(x)
+        hdn = linear(self.proj_in, x)
         ltxk.gelu_tanh(hdn, out=hdn)
         return linear(self.proj_out, hdn)

@@ -116,3 +116,31 @@ def test_layer_route(shape, n, bias, own):
         assert torch.equal(ltx_nn.linear(layer, x), want) and seen == [1]
         handle.remove()
     assert ltx_nn.linear(layer, x).requires_grad  # a recorded gradient keeps the layer's own call
+
+
+@pytest.mark.parametrize("m,n,k,main", [
+    (4096, 4096, 4096, 0), (4097, 4096, 4096, 4096), (4864, 4096, 2048, 4096), (4865, 4096, 2048, 0),
+    (8200, 4096, 16384, 8192), (5200, 16384, 4096, 5120), (1100, 16384, 4096, 0), (4290, 2048, 4096, 0),
+    (4290, 4096, 1024, 0), (4290, 12288, 4096, 0), (4290, 5000, 4096, 0), (4290, 4096, 188160, 0)])
+def test_full_wave_rows(m, n, k, main):
+    import ltx_nn
+
+    assert ltx_nn.full_wave_rows(m, n, k) == main
+
+
+@pytest.mark.parametrize("shape,bias", [((1, 4097), True), ((2, 2200), False)])
+def test_rows_past_a_full_wave(shape, bias):
+    """Both launches' rows against the product in fp64; a hooked layer keeps one call."""
+    import ltx_nn
+
+    layer = torch.nn.Linear(2048, 4096, bias=bias, device=DEV, dtype=torch.bfloat16)
+    x = torch.randn(*shape, 2048, device=DEV).to(torch.bfloat16)
+    m = x.numel() // 2048
+    assert ltx_nn.full_wave_rows(m, 4096, 2048) == 4096
+    with torch.no_grad():
+        got = ltx_nn.linear(layer, x)
+        assert got.shape == (*shape, 4096)
+        _check(x.view(m, 2048), layer.weight, layer.bias, got.view(m, 4096))
+        seen = []
+        layer.register_forward_hook(lambda *a: seen.append(1))
+        assert torch.equal(ltx_nn.linear(layer, x), layer(x)) and seen == [1, 1]
