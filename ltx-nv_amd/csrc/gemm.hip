@@ -6,7 +6,7 @@
 // What bounds it: the card's power and, with it, the loads beside the products.
 // [1024, 188160] x [4096, 188160] takes 1214-1236 us, 1.28-1.30 PFLOP/s (the
 // library's product, which leaves three of four compute units idle: 2100-2139 us,
-// 0.74-0.75), [4290, 16384] x [4096, 16384] 443-451 (843).  On zeros, 8192^3 runs at
+// 0.74-0.75), [512, 16384] x [4096, 16384] 73 (86).  On zeros, 8192^3 runs at
 // 1.72 PFLOP/s and 2.07 without its loads.  So:
 // * 256 x 256 tiles (half the loads of 128 x 256, which ran 15 % slower), eight
 //   waves of 128 x 64: four of 128 x 128 took 887 against 846 us on 8192^3.
