@@ -10,7 +10,7 @@
 // bf16 for the second product.
 //
 // What bounds it: the card's power.  On 6144 x 6144 tokens, 32 heads of 128, it
-// runs at 1.02-1.08 PFLOP/s (573-606 us by box) and the same launch on zeros,
+// runs at 1.01-1.08 PFLOP/s (573-612 us from card to card) and the same launch on zeros,
 // which switch nothing, at 1.63-1.66; torch's flash kernel 0.69 (865-916 us) on
 // the same inputs.  So the split is taken for the least work beside the products:
 // * Four waves of 32 queries share a 64-key tile in LDS (two workgroups a CU).
@@ -23,7 +23,7 @@
 // * V is read from LDS by transposing reads, so neither operand is rearranged.
 // * The second product of a tile and the scores of the next run as one stream,
 //   LDS fragments four ahead: 592-602 us with the products apart.  The loads of the
-//   next tile go between the products: 612 against 623 us (one box) with all of
+//   next tile go between the products: 612 against 623 us (one card) with all of
 //   them ahead of the stream, and without any loads (a timing copy) 11 % less.
 // * The running maximum is exact in every tile.  Letting it lag up to 2^8 saves
 //   2-4 %, but then a row's largest weight is no longer exactly 1 and its

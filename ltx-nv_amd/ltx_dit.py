@@ -18,7 +18,8 @@ elementwise ops share one pass over the activation:
   A2V/V2A inputs           both modulations of vx_pre (and of ax_pre) from
                            one read
   q/k norm + RoPE          one in-place launch for q and k
-  gate + head merge        one launch on the attention output
+  gate + head merge        inside the attention (one launch after it where a
+                           perturbation blends the values in)
 The flag reads of apply_block_perturbations use one host copy of the
 perturbation table per model call instead of three device syncs per block.
 """
