@@ -90,3 +90,39 @@ def test_strided_operands_and_refusals():
     assert call(head_dim=96) == ltxk.E_ARG and call(tk=0) == ltxk.E_ARG
     assert lib.ltxk_attention_workspace_bytes(b, t, 4096, h, dh) > 0
     assert call(tk=4096) == ltxk.E_ARG
+
+
+def test_captured_calls_replay_equal():
+    """Attention with cut keys, a linear layer cut over K and layers over few rows in
+    one captured graph: every replay, with other inputs and eager work between,
+    equals the eager calls bit for bit (their scratch comes from the graph's pool)."""
+    import ltxk
+
+    g = torch.Generator(device=DEV).manual_seed(9)
+
+    def fresh(*shape):
+        return torch.randn(*shape, device=DEV, generator=g).to(torch.bfloat16)
+
+    q, k, v, logits = fresh(1, 100, 256), fresh(1, 3000, 256), fresh(1, 3000, 256), fresh(1, 100, 4)
+    x, w, b = fresh(300, 16384), fresh(256, 16384) * 0.02, fresh(256)
+    few, few_w = fresh(70, 512), [fresh(64, 512), fresh(40, 512)]
+
+    def call():
+        return [ltxk.attention(q, k, v, 4, logits), ltxk.linear(x, w, b), *ltxk.linear_layers(few, few_w, [None, None])]
+
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        captured = call()
+    for _ in range(4):
+        for t in (q, k, v, logits, x, few):
+            t.copy_(fresh(*t.shape))
+        want = call()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, e in zip(captured, want):
+            assert torch.equal(a.view(torch.int16), e.view(torch.int16))
