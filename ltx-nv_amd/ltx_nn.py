@@ -334,15 +334,18 @@ def _plain_input(x: torch.Tensor) -> bool:
 
 def _plain_layer(layer: torch.nn.Linear, x: torch.Tensor) -> tuple | None:
     """(weight, bias) of a bare torch.nn.Linear (no hooks, its own forward, plain
-    tensors) whose operands fit x like _plain_input, else None.  Reads the module's
-    dictionaries: its attribute lookup costs more than the rest (`project` over
-    four layers takes the host 30 us with it, 16 without)."""
+    tensors) whose operands fit x like _plain_input, else None.  They must have the
+    layer's own shapes: torch broadcasts a bias of one entry, the kernels read
+    out_features of them.  Reads the module's dictionaries: its attribute lookup
+    costs more than the rest (`project` over four layers takes the host 30 us with
+    it, 16 without)."""
     if type(layer) is not torch.nn.Linear or layer._forward_hooks or layer._forward_pre_hooks \
             or "forward" in layer.__dict__ or _has_any_global_hook():
         return None
     params = layer._parameters
     w, b = params.get("weight"), params.get("bias")
-    if w is None or w.shape[1] != x.shape[-1]:
+    n = layer.out_features
+    if w is None or w.shape != (n, x.shape[-1]) or (b is not None and b.shape != (n,)):
         return None
     for t in (w, b):
         if t is not None and not (type(t) in (torch.nn.Parameter, torch.Tensor) and t.get_device() == x.get_device()

@@ -1,0 +1,40 @@
+"""Which calls ltx_nn hands to the matrix-core entry points and which stay with
+torch: the rules that need no GPU."""
+
+import pytest
+import torch
+
+BF16 = torch.bfloat16
+
+
+def _layer(k=128, n=64, bias=True):
+    return torch.nn.Linear(k, n, bias=bias, dtype=BF16).requires_grad_(False)
+
+
+def _param(*shape):
+    return torch.nn.Parameter(torch.zeros(*shape, dtype=BF16), requires_grad=False)
+
+
+def test_layer_of_its_own_shapes_is_plain():
+    import ltx_nn
+
+    x = torch.zeros(3, 128, dtype=BF16)
+    layer = _layer()
+    weight, bias = ltx_nn._plain_layer(layer, x)
+    assert weight is layer.weight and bias is layer.bias
+    assert ltx_nn._plain_layer(_layer(bias=False), x)[1] is None
+
+
+@pytest.mark.parametrize("weight,bias", [
+    ((64, 128), (1,)), ((64, 128), (32,)), ((64, 128), (128,)), ((64, 128), (64, 1)), ((64, 128), (1, 64)),
+    ((40, 128), (64,)), ((60, 128), (60,)), ((128,), (64,)), ((128,), None), ((64, 64), (64,))])
+def test_layer_of_other_shapes_keeps_torch(weight, bias):
+    """A replaced weight or bias whose shape is not the layer's own (torch broadcasts
+    some of them and refuses the others) is not handed to kernels that read
+    out_features entries of it."""
+    import ltx_nn
+
+    layer = _layer()
+    layer.weight = _param(*weight)
+    layer.bias = None if bias is None else _param(*bias)
+    assert ltx_nn._plain_layer(layer, torch.zeros(3, 128, dtype=BF16)) is None
