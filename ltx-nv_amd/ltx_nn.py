@@ -332,6 +332,9 @@ def _plain_input(x: torch.Tensor) -> bool:
         and not (torch.is_grad_enabled() and x.requires_grad) and not torch.is_autocast_enabled("cuda")
 
 
+_OWN_ATTRIBUTES = {"forward", "weight", "bias"}  # set on a layer itself, these come before its class and parameters
+
+
 def _plain_layer(layer: torch.nn.Linear, x: torch.Tensor) -> tuple | None:
     """(weight, bias) of a bare torch.nn.Linear (no hooks, its own forward, plain
     tensors) whose operands fit x like _plain_input, else None.  They must have the
@@ -340,12 +343,12 @@ def _plain_layer(layer: torch.nn.Linear, x: torch.Tensor) -> tuple | None:
     costs more than the rest (`project` over four layers takes the host 30 us with
     it, 16 without)."""
     if type(layer) is not torch.nn.Linear or layer._forward_hooks or layer._forward_pre_hooks \
-            or "forward" in layer.__dict__ or _has_any_global_hook():
+            or _OWN_ATTRIBUTES & layer.__dict__.keys() or _has_any_global_hook():
         return None
     params = layer._parameters
     w, b = params.get("weight"), params.get("bias")
     n = layer.out_features
-    if w is None or w.shape != (n, x.shape[-1]) or (b is not None and b.shape != (n,)):
+    if w is None or "bias" not in params or w.shape != (n, x.shape[-1]) or (b is not None and b.shape != (n,)):
         return None
     for t in (w, b):
         if t is not None and not (type(t) in (torch.nn.Parameter, torch.Tensor) and t.get_device() == x.get_device()

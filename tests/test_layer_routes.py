@@ -38,3 +38,21 @@ def test_layer_of_other_shapes_keeps_torch(weight, bias):
     layer.weight = _param(*weight)
     layer.bias = None if bias is None else _param(*bias)
     assert ltx_nn._plain_layer(layer, torch.zeros(3, 128, dtype=BF16)) is None
+
+
+@pytest.mark.parametrize("name", ["weight", "bias"])
+@pytest.mark.parametrize("where", ["attribute", "buffer", "shadow"])
+def test_operand_kept_elsewhere_keeps_torch(name, where):
+    """A layer whose weight or bias is not (or not only) among its parameters: torch
+    reads the attribute, so the parameter dictionary alone does not name the operand."""
+    import ltx_nn
+
+    layer = _layer()
+    value = torch.ones_like(getattr(layer, name).data)
+    if where == "shadow":
+        object.__setattr__(layer, name, value)
+    else:
+        delattr(layer, name)
+        layer.register_buffer(name, value) if where == "buffer" else setattr(layer, name, value)
+    assert getattr(layer, name) is value
+    assert ltx_nn._plain_layer(layer, torch.zeros(3, 128, dtype=BF16)) is None
