@@ -56,3 +56,30 @@ def test_operand_kept_elsewhere_keeps_torch(name, where):
         layer.register_buffer(name, value) if where == "buffer" else setattr(layer, name, value)
     assert getattr(layer, name) is value
     assert ltx_nn._plain_layer(layer, torch.zeros(3, 128, dtype=BF16)) is None
+
+
+@pytest.mark.parametrize("m,k,widths,taken", [
+    (1, 128, (8, 2**24 - 8), True), (1, 128, (8, 2**24), False), (4, 128, (2**24 + 8, 8), False),
+    (4096, 128, (2**19 - 8, 8), True), (4096, 128, (8, 2**19), False), (126, 2048, (2048, 2048, 2048, 32), True),
+    (126, 2048, (2048, 36), False)])
+def test_few_rows_widths(m, k, widths, taken):
+    """Layers that ltxk_linear_layers refuses keep torch's call."""
+    import ltx_nn
+
+    assert ltx_nn.few_rows_widths(m, k, widths) == taken
+
+
+def test_few_rows_of_a_huge_layer_keep_torch(monkeypatch):
+    import ltx_nn
+    import ltxk
+
+    class Huge(torch.nn.Module):  # stands for a layer of 2^24 + 8 rows of 128, which has no memory here
+        def forward(self, x):
+            return x.new_zeros(x.shape[0], 8)
+
+    layers = [Huge(), Huge()]
+    weight = torch.empty(2**24 + 8, 128, dtype=BF16, device="meta")
+    monkeypatch.setattr(ltx_nn, "_plain_input", lambda x: True)
+    monkeypatch.setattr(ltx_nn, "_plain_layer", lambda layer, x: (weight, None))
+    monkeypatch.setattr(ltxk, "_launch_layers", lambda *a: pytest.fail("launched"))
+    assert [y.shape for y in ltx_nn.project(torch.zeros(2, 128, dtype=BF16), *layers)] == [(2, 8)] * 2
