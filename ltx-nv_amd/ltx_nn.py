@@ -396,13 +396,19 @@ def _two_launches(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | No
 FEW_ROWS_MAX = 1 << 19
 
 
+def few_rows_widths(m: int, k: int, widths) -> bool:
+    """Whether ltxk_linear_layers takes layers of these widths over m rows of k: each
+    a multiple of 8, weights and outputs of fewer than 2^31 elements."""
+    return all(n % 8 == 0 and max(m, k) * n < 2**31 for n in widths)
+
+
 def project(x: torch.Tensor, *layers: torch.nn.Linear | None) -> list:
     """[layer(x) for each layer], None for None, in one launch where x is small."""
     real = [layer for layer in layers if layer is not None]
     if 2 <= len(real) <= ltxk.MAX_LINEAR_LAYERS and x.numel() <= FEW_ROWS_MAX and x.shape[-1] % 128 == 0 \
             and _plain_input(x):
-        plain = [_plain_layer(layer, x) for layer in real]
-        if all(p is not None and p[0].shape[0] % 8 == 0 for p in plain):
+        plain, k = [_plain_layer(layer, x) for layer in real], x.shape[-1]
+        if None not in plain and few_rows_widths(x.numel() // k, k, [w.shape[0] for w, _ in plain]):
             weights, biases = zip(*plain)
             done = iter(ltxk._launch_layers(x, weights, biases))
             return [None if layer is None else next(done) for layer in layers]
