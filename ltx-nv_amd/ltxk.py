@@ -405,7 +405,10 @@ def _launch_limits(index: int) -> tuple[int, int]:
 def device_policy_threads(n: int, device: torch.device | int | None = None) -> int:
     """T that torch's grid-stride launch policy picks for n values on `device`."""
     if device is not None and not isinstance(device, int):
-        device = torch.device(device).index
+        device = torch.device(device)
+        if device.type != "cuda":
+            raise ValueError(f"expected a GPU, got {device}")
+        device = device.index
     return policy_threads(n, *_launch_limits(device if device is not None else torch.cuda.current_device()))
 
 

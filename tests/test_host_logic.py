@@ -174,3 +174,17 @@ def test_patchify_layouts_and_round_trips():
     assert torch.equal(ta, rearrange(a, "b c t m -> b t (c m)"))
     assert torch.equal(ta[0, 6, 3 * 16 + 9], a[0, 3, 6, 9])
     assert torch.equal(ltx_dit.unpatchify_audio(ta, 8, 16), a)
+
+
+def test_policy_threads_of_a_device_that_is_no_gpu_are_refused(monkeypatch):
+    """As torch.cuda.get_device_properties refuses it, instead of answering for the
+    current GPU; a GPU without an index is the current one."""
+    import ltxk
+
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(ltxk, "_launch_limits", lambda index: {0: (256, 2048), 1: (142, 1536)}[index])
+    for device in ("cpu", "cpu:0", torch.device("cpu"), "meta"):
+        with pytest.raises(ValueError):
+            ltxk.device_policy_threads(1 << 28, device)
+    for device, limits in ((None, (256, 2048)), ("cuda", (256, 2048)), ("cuda:1", (142, 1536)), (1, (142, 1536))):
+        assert ltxk.device_policy_threads(1 << 28, device) == ltxk.policy_threads(1 << 28, *limits)
