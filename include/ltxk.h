@@ -365,10 +365,11 @@ int64_t ltxk_attention_workspace_bytes(int64_t batch, int64_t tokens_q, int64_t 
  * q is bf16 at q + b*q_bstride + t*q_tstride + h*head_dim (elements, multiples
  * of 8, token strides at least heads*head_dim), k and v likewise; out is
  * contiguous token-major [batch*tokens_q, heads*head_dim], logits contiguous
- * [batch*tokens_q, heads].  Scores, softmax and sums are fp32, the weights
- * bf16 in the product with v.  The keys of one batch item span less than 2^31
- * bytes.  `workspace`: device memory of ltxk_attention_workspace_bytes, 16-byte
- * aligned (NULL if that is 0), in use until the call's work has run.
+ * [batch*tokens_q, heads].  scale is positive, and finite also times log2(e).
+ * Scores, softmax and sums are fp32, the weights bf16 in the product with v.
+ * The keys of one batch item span less than 2^31 bytes.  `workspace`: device
+ * memory of ltxk_attention_workspace_bytes, 16-byte aligned (NULL if that is 0),
+ * in use until the call's work has run.
  * Replaces SDPA, the head merge and the gate (standalone/ltx_nn.py:22-26,
  * 227-235). */
 int ltxk_attention(void *out, const void *q, int64_t q_bstride, int64_t q_tstride, const void *k, int64_t k_bstride,

@@ -30,6 +30,7 @@
 //   rounding shows: relative error 2.26e-3 against 1.87e-3 (torch's 1.87e-3).
 #include "ltxk_common.h"
 
+#include <cfloat>
 #include <type_traits>
 
 namespace ltxk {
@@ -432,6 +433,10 @@ extern "C" int ltxk_attention(void *out, const void *q, int64_t q_bstride, int64
         return fail(LTXK_E_ARG, "%s: head_dim must be 64 or 128 (got %lld)", what, (long long)head_dim);
     if (batch == 0 || tokens_q == 0) return LTXK_OK;
     if (tokens_k == 0) return fail(LTXK_E_ARG, "%s: no keys", what);
+    // the maximum is taken of the raw scores, and keys past the last are closed with -inf before the scaling
+    const float scale2 = scale * 1.4426950408889634f;
+    if (!(scale > 0.f && scale2 <= FLT_MAX))
+        return fail(LTXK_E_ARG, "%s: scale must be positive and finite (got %g)", what, static_cast<double>(scale));
     if (!out || !q || !k || !v) return fail(LTXK_E_ARG, "%s: null out, q, k or v", what);
     if (!aligned16(out) || !aligned16(q) || !aligned16(k) || !aligned16(v) ||
         (reinterpret_cast<uintptr_t>(logits) & 1u))
@@ -475,7 +480,7 @@ extern "C" int ltxk_attention(void *out, const void *q, int64_t q_bstride, int64
     p.whole = static_cast<int>(c.whole);
     p.rest = static_cast<int>(c.rest);
     p.parts = static_cast<int>(c.parts);
-    p.scale2 = scale * 1.4426950408889634f;
+    p.scale2 = scale2;
     if (head_dim == 128)
         launch<128>(p, static_cast<hipStream_t>(stream));
     else

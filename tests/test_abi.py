@@ -187,3 +187,18 @@ def test_noalloc_guide_rejects_oversize_before_any_device_call():
     rc = lib.ltxk_guide_noalloc(p, None, None, p, p, None, 0, 0, (1 << 28) // 64 + 1, 64, ctypes.byref(gp), 0.5,
                                 -0.1, None)
     assert rc == ltxk.E_ARG and "2^28" in ltxk.last_error()
+
+
+@pytest.mark.parametrize("scale", [0.0, -0.125, float("nan"), float("inf"), -float("inf"), 3e38])
+def test_attention_refuses_scales_without_a_softmax_of_the_maximum(scale):
+    """Scales that are not positive, or not finite in the kernel's base-2 form: its
+    running maximum is the scaled maximum of the raw scores.  Refused before any
+    launch (the pointers are never dereferenced)."""
+    import ltxk
+
+    lib = ltxk.load()
+    p = ctypes.c_void_p(256)
+    # rows of 2^31 bytes: refused by their size too, after the scale
+    rc = lib.ltxk_attention(p, p, 64, 64, p, 1 << 30, 1 << 30, p, 1 << 30, 1 << 30, None, 1, 20, 20, 1, 64, scale,
+                            None, 0, None)
+    assert rc == ltxk.E_ARG and "scale" in ltxk.last_error()
