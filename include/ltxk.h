@@ -382,22 +382,23 @@ int64_t ltxk_linear_workspace_bytes(int64_t m, int64_t n, int64_t k);
 
 /* y = round(x w^T + bias) for bf16 x [m, k], w [n, k], y [m, n], bias [n] or NULL,
  * all contiguous and 16-byte aligned; fp32 sums, bias added in fp32, one
- * rounding.  n is a multiple of 8, k of 64; x, w and y hold at most 2^31
- * elements each.  Output tiles past the last full wave of the chip are cut over
- * k, their fp32 sums held in `workspace` (ltxk_linear_workspace_bytes, 16-byte
- * aligned; NULL if that is 0).  For the projections that a library product
- * leaves to few compute units: the feature extractor's (k = 188160,
- * standalone/ltx_te.py:179-184) and the FFN's second one (ltx_nn.py:247-248). */
+ * rounding.  n is a multiple of 8, k of 64; x and w hold fewer than 2^31
+ * elements each, y at most 2^31.  Output tiles past the last full wave of the
+ * chip are cut over k, their fp32 sums held in `workspace`
+ * (ltxk_linear_workspace_bytes, 16-byte aligned; NULL if that is 0).  For the
+ * projections that a library product leaves to few compute units: the feature
+ * extractor's (k = 188160, standalone/ltx_te.py:179-184) and the FFN's second one
+ * (ltx_nn.py:247-248). */
 int ltxk_linear(void *y, const void *x, const void *w, const void *bias, int64_t m, int64_t n, int64_t k,
                 void *workspace, int64_t workspace_bytes, void *stream);
 
 /* y[i] = round(x w[i]^T + bias[i]) for 1 to 4 layers over the same few rows x
  * [m, k], in one launch: w[i] [n[i], k], y[i] [m, n[i]], bias[i] [n[i]] (or NULL,
  * as `bias` itself), bf16, contiguous, 16-byte aligned; fp32 sums, one rounding.
- * n[i] is a multiple of 8, k of 128; x and each w and y hold at most 2^31
- * elements.  y, w, bias and n are host arrays.  For the projections of one
- * attention's input (standalone/ltx_nn.py:188-192,205-207) over an audio stream's
- * rows. */
+ * n[i] is a multiple of 8, k of 128; x and each w hold fewer than 2^31 elements,
+ * each y at most 2^31.  y, w, bias and n are host arrays.  For the projections of
+ * one attention's input (standalone/ltx_nn.py:188-192,205-207) over an audio
+ * stream's rows. */
 int ltxk_linear_layers(void *const *y, const void *x, const void *const *w, const void *const *bias,
                        const int64_t *n, int64_t layers, int64_t m, int64_t k, void *stream);
 

@@ -390,10 +390,10 @@ extern "C" int ltxk_linear(void *y, const void *x, const void *w, const void *bi
     if (!y || !x || !w) return fail(LTXK_E_ARG, "%s: null y, x or w", what);
     if (!aligned16(y) || !aligned16(x) || !aligned16(w) || !aligned16(bias))
         return fail(LTXK_E_ALIGN, "%s: y, x, w and bias must be 16-byte aligned", what);
-    // operands are addressed with 32-bit byte offsets, outputs by 32-bit tile counts
+    // operands are read through descriptors of 2^32 - 1 bytes, outputs counted by 32-bit tiles
     const int64_t kMax = int64_t{1} << 31;
-    if (k >= kMax / 2 || m > kMax / k || n > kMax / k || m > kMax / n)
-        return fail(LTXK_E_ARG, "%s: x, w or y spans 2^32 bytes or more", what);
+    if (k >= kMax / 2 || m > (kMax - 1) / k || n > (kMax - 1) / k || m > kMax / n)
+        return fail(LTXK_E_ARG, "%s: x or w holds 2^31 elements or more, or y more than 2^31", what);
     GemmParams p{};
     p.x = static_cast<const uint16_t *>(x);
     p.w = static_cast<const uint16_t *>(w);
@@ -433,7 +433,7 @@ extern "C" int ltxk_linear_layers(void *const *y, const void *x, const void *con
     const int64_t kMax = int64_t{1} << 31;
     if (!x) return fail(LTXK_E_ARG, "%s: null x", what);
     if (!aligned16(x)) return fail(LTXK_E_ALIGN, "%s: x must be 16-byte aligned", what);
-    if (k >= kMax / 2 || m > kMax / k) return fail(LTXK_E_ARG, "%s: x spans 2^32 bytes or more", what);
+    if (k >= kMax / 2 || m > (kMax - 1) / k) return fail(LTXK_E_ARG, "%s: x holds 2^31 elements or more", what);
     FewParams p{};
     p.x = static_cast<const uint16_t *>(x);
     p.m = static_cast<int>(m);
@@ -447,9 +447,12 @@ extern "C" int ltxk_linear_layers(void *const *y, const void *x, const void *con
             continue;
         }
         const void *b = bias ? bias[i] : nullptr;
-        if (n[i] <= 0 || n[i] % 8 || n[i] > kMax / k || m > kMax / n[i])
-            return fail(LTXK_E_ARG, "%s: layer %lld: n must be a positive multiple of 8 within 2^31 elements (got %lld)",
-                        what, (long long)i, (long long)n[i]);
+        if (n[i] <= 0 || n[i] % 8)
+            return fail(LTXK_E_ARG, "%s: layer %lld: n must be a positive multiple of 8 (got %lld)", what, (long long)i,
+                        (long long)n[i]);
+        if (n[i] > (kMax - 1) / k || m > kMax / n[i])
+            return fail(LTXK_E_ARG, "%s: layer %lld: w holds 2^31 elements or more, or y more than 2^31", what,
+                        (long long)i);
         if (!y[i] || !w[i]) return fail(LTXK_E_ARG, "%s: layer %lld: null y or w", what, (long long)i);
         if (!aligned16(y[i]) || !aligned16(w[i]) || !aligned16(b))
             return fail(LTXK_E_ALIGN, "%s: layer %lld: y, w and bias must be 16-byte aligned", what, (long long)i);

@@ -202,3 +202,21 @@ def test_attention_refuses_scales_without_a_softmax_of_the_maximum(scale):
     rc = lib.ltxk_attention(p, p, 64, 64, p, 1 << 30, 1 << 30, p, 1 << 30, 1 << 30, None, 1, 20, 20, 1, 64, scale,
                             None, 0, None)
     assert rc == ltxk.E_ARG and "scale" in ltxk.last_error()
+
+
+def test_products_of_two_to_the_31_elements_are_refused():
+    """The products read x and the weights through descriptors of 2^32 - 1 bytes, one
+    less than 2^31 elements span: refused before any launch."""
+    import ltxk
+
+    lib = ltxk.load()
+    p = ctypes.c_void_p(256)
+    for m, n, k in ((1 << 15, 8, 1 << 16), (8, 1 << 15, 1 << 16)):
+        # without the workspace that these shapes need: refused for that, too
+        assert lib.ltxk_linear(p, p, p, None, m, n, k, None, 0, None) == ltxk.E_ARG
+        assert "2^31" in ltxk.last_error()
+    ptrs, empty = (ctypes.c_void_p * 2)(256, 256), (ctypes.c_void_p * 2)(256, None)
+    for m, n, k in ((1 << 24, 8, 128), (8, 1 << 24, 128)):
+        # the second layer has no weight
+        rc = lib.ltxk_linear_layers(ptrs, p, empty, None, (ctypes.c_int64 * 2)(n, 8), 2, m, k, None)
+        assert rc == ltxk.E_ARG and "2^31" in ltxk.last_error()
