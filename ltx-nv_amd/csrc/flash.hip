@@ -452,7 +452,8 @@ extern "C" int ltxk_attention(void *out, const void *q, int64_t q_bstride, int64
         (tokens_k + kKeys) > kMax / 2 / v_tstride)
         return fail(LTXK_E_ARG, "%s: a batch item's keys or values span 2^31 bytes or more", what);
     const FlashCut c = cut(batch * heads, tokens_q, tokens_k);
-    if ((c.whole + c.rest * c.parts) > (1 << 28) || c.q_tiles > kMax / 8)
+    // a launch holds fewer than 2^32 threads
+    if (c.whole + c.rest * c.parts >= (int64_t{1} << 32) / (8 * kWaves * 64))
         return fail(LTXK_E_ARG, "%s: too many query tiles", what);
     if (c.rest && (!workspace || !aligned16(workspace) ||
                    workspace_bytes < ltxk_attention_workspace_bytes(batch, tokens_q, tokens_k, heads, head_dim)))

@@ -77,14 +77,21 @@ def key_split_partials(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, parts:
     return out, lse
 
 
+def attention_grid_fits(batch: int, tokens: int, heads: int) -> bool:
+    """Whether ltxk_attention's launch holds these queries: at most 2^20 batch items,
+    and fewer than 2^21 tiles of 128 queries on each of the 8 XCDs (2^32 threads),
+    with room for the 64 units that cut keys make there."""
+    return batch <= 1 << 20 and -(-batch * heads // 8) * -(-tokens // 128) < (1 << 21) - 64
+
+
 def fused_attention_applies(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, heads: int, dim_head: int) -> bool:
     """Whether unmasked attention of token-major q over k, v runs on
     ltxk_attention: contiguous 16-byte aligned bf16 tensors on one ROCm device,
     heads of 64 or 128, keys of one batch item within the kernel's 32-bit
-    offsets, and no gradient to record."""
+    offsets, queries within its launch, and no gradient to record."""
     if not (dim_head in ltxk.ATTENTION_HEAD_DIMS and q.ndim == k.ndim == 3 and v.shape == k.shape
             and q.shape[0] == k.shape[0] and q.shape[2] == k.shape[2] == heads * dim_head and k.shape[1] > 0
-            and (k.shape[1] + 64) * k.shape[2] < 2**30):
+            and (k.shape[1] + 64) * k.shape[2] < 2**30 and attention_grid_fits(q.shape[0], q.shape[1], heads)):
         return False
     if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):
         return False

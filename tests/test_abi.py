@@ -220,3 +220,17 @@ def test_products_of_two_to_the_31_elements_are_refused():
         # the second layer has no weight
         rc = lib.ltxk_linear_layers(ptrs, p, empty, None, (ctypes.c_int64 * 2)(n, 8), 2, m, k, None)
         assert rc == ltxk.E_ARG and "2^31" in ltxk.last_error()
+
+
+def test_attention_refuses_grids_past_the_launch_limit():
+    """2^21 query tiles an XCD are 2^32 threads, one too many for a launch: refused
+    as an argument before it."""
+    import ltxk
+
+    lib = ltxk.load()
+    p = ctypes.c_void_p(256)
+    for batch, tokens, heads in ((1 << 20, 1, 16), (1, 1 << 28, 8), (1 << 18, 129, 32)):
+        width = heads * 64
+        rc = lib.ltxk_attention(p, p, tokens * width, width, p, width, width, p, width, width, None, batch, tokens, 1,
+                                heads, 64, 0.125, None, 0, None)
+        assert rc == ltxk.E_ARG and "too many query tiles" in ltxk.last_error()

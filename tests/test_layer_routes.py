@@ -83,3 +83,13 @@ def test_few_rows_of_a_huge_layer_keep_torch(monkeypatch):
     monkeypatch.setattr(ltx_nn, "_plain_layer", lambda layer, x: (weight, None))
     monkeypatch.setattr(ltxk, "_launch_layers", lambda *a: pytest.fail("launched"))
     assert [y.shape for y in ltx_nn.project(torch.zeros(2, 128, dtype=BF16), *layers)] == [(2, 8)] * 2
+
+
+@pytest.mark.parametrize("batch,tokens,heads,fits", [
+    (1, 6144, 32, True), (1 << 20, 1, 8, True), ((1 << 20) + 1, 1, 1, False), (1 << 20, 1, 16, False),
+    (1 << 19, 128, 16, True), (1 << 19, 129, 16, False), (1, (1 << 28) - (1 << 14), 8, True), (1, 1 << 28, 8, False)])
+def test_attention_grid_fits(batch, tokens, heads, fits):
+    """Batches and query counts past ltxk_attention's launch keep torch's attention."""
+    import ltx_nn
+
+    assert ltx_nn.attention_grid_fits(batch, tokens, heads) == fits
