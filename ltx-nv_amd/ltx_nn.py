@@ -17,6 +17,7 @@ import math
 import numpy
 import torch
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 from torch.nn.attention import SDPBackend, sdpa_kernel
 from torch.nn.modules.module import _has_any_global_hook
 
@@ -77,6 +78,14 @@ def key_split_partials(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, parts:
     return out, lse
 
 
+def eager_call() -> bool:
+    """Whether operations just run as they are called: no tracer, function transform,
+    forward-mode derivative or dispatch mode is to see them.  The ltxk entry points
+    bypass torch's dispatcher, so calls that one watches keep torch's operations."""
+    return not (torch._C._len_torch_dispatch_stack() or torch._C._is_tracing() or forward_ad._current_level >= 0
+                or torch._C._functorch.peek_interpreter_stack() is not None or torch.compiler.is_compiling())
+
+
 def attention_grid_fits(batch: int, tokens: int, heads: int) -> bool:
     """Whether ltxk_attention's launch holds these queries: at most 2^20 batch items,
     and fewer than 2^21 tiles of 128 queries on each of the 8 XCDs (2^32 threads),
@@ -88,12 +97,13 @@ def fused_attention_applies(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, h
     """Whether unmasked attention of token-major q over k, v runs on
     ltxk_attention: contiguous 16-byte aligned bf16 tensors on one ROCm device,
     heads of 64 or 128, keys of one batch item within the kernel's 32-bit
-    offsets, queries within its launch, and no gradient to record."""
+    offsets, queries within its launch, no gradient to record and an
+    eager call."""
     if not (dim_head in ltxk.ATTENTION_HEAD_DIMS and q.ndim == k.ndim == 3 and v.shape == k.shape
             and q.shape[0] == k.shape[0] and q.shape[2] == k.shape[2] == heads * dim_head and k.shape[1] > 0
             and (k.shape[1] + 64) * k.shape[2] < 2**30 and attention_grid_fits(q.shape[0], q.shape[1], heads)):
         return False
-    if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):
+    if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad) or not eager_call():
         return False
     return all(t.is_cuda and t.device == q.device and t.dtype == torch.bfloat16 and t.is_contiguous()
                and t.data_ptr() % 16 == 0 for t in (q, k, v))
@@ -334,9 +344,9 @@ def full_wave_rows(m: int, n: int, k: int) -> int:
 
 def _plain_input(x: torch.Tensor) -> bool:
     """Whether the ltxk products can read x: contiguous aligned bf16 on a ROCm
-    device, no autocast, no gradient to record."""
-    return x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous() and x.data_ptr() % 16 == 0 and x.numel() > 0 \
-        and not (torch.is_grad_enabled() and x.requires_grad) and not torch.is_autocast_enabled("cuda")
+    device, no autocast, no gradient to record, an eager call."""
+    return x.is_cuda and x.dtype == torch.bfloat16 and eager_call() and x.is_contiguous() and x.data_ptr() % 16 == 0 \
+        and x.numel() > 0 and not (torch.is_grad_enabled() and x.requires_grad) and not torch.is_autocast_enabled("cuda")
 
 
 _OWN_ATTRIBUTES = {"forward", "weight", "bias"}  # set on a layer itself, these come before its class and parameters

@@ -126,3 +126,22 @@ def test_captured_calls_replay_equal():
         torch.cuda.synchronize()
         for a, e in zip(captured, want):
             assert torch.equal(a.view(torch.int16), e.view(torch.int16))
+
+
+def test_attend_under_a_transform_and_a_mode():
+    """Attention.attend without gates, masks and hooks is torch operations under
+    vmap and under a dispatch mode that counts them, and gives what eager calls do."""
+    from torch.utils.flop_counter import FlopCounterMode
+
+    import ltx_nn
+
+    layer = ltx_nn.Attention(256, 256, 4, 64).to(device=DEV, dtype=torch.bfloat16).requires_grad_(False)
+    g = torch.Generator(device=DEV).manual_seed(3)
+    q, k, v = (torch.randn(3, 2, 70, 256, device=DEV, generator=g).to(torch.bfloat16) for _ in range(3))
+    want = torch.stack([layer.attend(*t, None) for t in zip(q, k, v)]).float()
+    got = torch.func.vmap(lambda *t: layer.attend(*t, None))(q, k, v).float()
+    # the attention's bf16 roundings and the output's
+    assert ((got - want).norm() / want.norm()).item() < 2.0**-7
+    with FlopCounterMode(display=False) as counted:
+        layer.attend(q[0], k[0], v[0], None)
+    assert counted.get_total_flops() >= 2 * 2 * 70 * 256 * (70 + 70 + 256)

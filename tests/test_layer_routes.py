@@ -93,3 +93,32 @@ def test_attention_grid_fits(batch, tokens, heads, fits):
     import ltx_nn
 
     assert ltx_nn.attention_grid_fits(batch, tokens, heads) == fits
+
+
+def test_calls_that_torch_watches_are_no_eager_calls():
+    """Tracing, function transforms, forward-mode derivatives and dispatch modes see
+    only torch's own operations, so calls under them keep those."""
+    from torch.autograd import forward_ad
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.utils.flop_counter import FlopCounterMode
+
+    import ltx_nn
+
+    seen = []
+
+    def call(x):
+        seen.append(ltx_nn.eager_call())
+        return x * 2
+
+    x = torch.ones(2, 3)
+    torch.func.vmap(call)(x)
+    torch.func.grad(lambda t: call(t).sum())(x)
+    torch.func.jvp(call, (x,), (x,))
+    torch.jit.trace(call, x, check_trace=False)
+    make_fx(call)(x)
+    with FlopCounterMode(display=False):
+        call(x)
+    with forward_ad.dual_level():
+        call(forward_ad.make_dual(x, x))
+    assert len(seen) >= 7 and not any(seen)
+    assert ltx_nn.eager_call()
