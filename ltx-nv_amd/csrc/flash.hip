@@ -43,11 +43,13 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int kWaves = 4;
 constexpr int kRows = 32 * kWaves;  // queries a workgroup, 32 a wave
 constexpr int kKeys = 64;           // keys a tile
+constexpr float kLarge = 4096.f;    // scaled scores whose products' rounding the weights may show
 
 struct FlashParams {
     const uint16_t *q, *k, *v, *logits;
     uint16_t *out;
-    float *part, *lse;      // split query tiles: each unit's output (128 x D) and log2-sum-exps (128)
+    float *part;            // split query tiles: each unit's weighted sums of v (128 x D)
+    float2 *stats;          // and each of its rows' maximum and sum of weights (128)
     int64_t qbs, kbs, vbs;  // batch strides, elements
     uint32_t qts, kts, vts; // token strides, bytes
     int tq, tk, heads, q_tiles, tiles;
@@ -200,7 +202,7 @@ __global__ void __launch_bounds__(kWaves * 64, 2) flash_kernel(FlashParams p)
     f32x16 o[MT] = {};
     f32x16 s[2];     // scores, transposed: register r of s[u] is key 32 u + 8 (r/4) + 4 half + r % 4 of query l % 32
     u32x4 w[4];      // weights, two a register, in the order of the scores
-    float mx = 0.f;  // running maximum times scale2 (the same in lanes l and l ^ 32)
+    float mx = 0.f;  // running maximum of the scaled scores (the same in lanes l and l ^ 32)
     float sum = 0.f; // this lane's share of the weights' sum
 
     // Fragment i of a K tile (contraction step i / 2 of keys 32 (i%2) ..) and of a
@@ -259,7 +261,7 @@ __global__ void __launch_bounds__(kWaves * 64, 2) flash_kernel(FlashParams p)
         }
         const float m = pair_max(fmaxf(fmaxf(t[0], t[1]), fmaxf(t[2], t[3]))) * p.scale2;
         if (i == 0) {
-            mx = fmaxf(m, -1e30f);  // finite, so that scores of -inf weigh zero
+            mx = fmaxf(m, -FLT_MAX);  // finite, so that scores of -inf weigh zero
         } else if (__any(m > mx)) {
             const float nm = fmaxf(m, mx);
             const float a = __builtin_amdgcn_exp2f(mx - nm);
@@ -270,11 +272,23 @@ __global__ void __launch_bounds__(kWaves * 64, 2) flash_kernel(FlashParams p)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) o[c][r] *= a;
         }
+        // The maximum is a rounded product and the scores' products below are exact, so
+        // the largest weight is 2^(a rounding of the maximum) instead of 1: past kLarge
+        // that would come to show in bf16 (and past 2^31 overflow), so there the scores
+        // round first (0.5 % of the time at 6144 tokens for the test).
+        float scale2 = p.scale2;
+        if (__any(fabsf(mx) > kLarge)) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) s[u][r] *= scale2;
+            scale2 = 1.f;
+        }
         float part[2] = {};
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
-            const float x = __builtin_amdgcn_exp2f(__builtin_fmaf(s[j >> 3][2 * (j & 7)], p.scale2, -mx));
-            const float y = __builtin_amdgcn_exp2f(__builtin_fmaf(s[j >> 3][2 * (j & 7) + 1], p.scale2, -mx));
+            const float x = __builtin_amdgcn_exp2f(__builtin_fmaf(s[j >> 3][2 * (j & 7)], scale2, -mx));
+            const float y = __builtin_amdgcn_exp2f(__builtin_fmaf(s[j >> 3][2 * (j & 7) + 1], scale2, -mx));
             part[0] += x;
             part[1] += y;
             w[j >> 2][j & 3] = pack_bf16x2(x, y);
@@ -313,19 +327,18 @@ __global__ void __launch_bounds__(kWaves * 64, 2) flash_kernel(FlashParams p)
 
     // Lane l: query l % 32, columns 32 m + 8 j + 4 half + (0..3) in registers 4 j ..
     const float total = pair_sum(sum);
-    const float inv = 1.f / total;
     if (split) {
-        const float pi = total == 0.f ? 0.f : inv;  // a unit whose scores are all -inf
         const int64_t u = (static_cast<int64_t>(xcd) * p.rest * p.parts + unit) * kRows + wave * 32 + l32;
-        if (half == 0) p.lse[u] = mx + __log2f(total);
+        if (half == 0) p.stats[u] = make_float2(mx, total);
 #pragma unroll
         for (int t = 0; t < MT; ++t)
 #pragma unroll
             for (int c = 0; c < 4; ++c)
                 *reinterpret_cast<f32x4 *>(p.part + u * D + 32 * t + 8 * c + 4 * half) =
-                    f32x4{o[t][4 * c] * pi, o[t][4 * c + 1] * pi, o[t][4 * c + 2] * pi, o[t][4 * c + 3] * pi};
+                    f32x4{o[t][4 * c], o[t][4 * c + 1], o[t][4 * c + 2], o[t][4 * c + 3]};
         return;
     }
+    const float inv = 1.f / total;
     if (row >= p.tq) return;
     const int64_t tok = (static_cast<int64_t>(b) * p.tq + row) * p.heads + head;
     const float gate = p.logits ? head_gate(p.logits[tok]) : 1.f;
@@ -353,13 +366,14 @@ __global__ void __launch_bounds__(256) flash_merge_kernel(FlashParams p)
     if (!query_tile(p, xcd, p.whole + t, b, head, first) || first + r >= p.tq) return;
     const int64_t u = (static_cast<int64_t>(xcd) * p.rest + t) * p.parts * kRows + r;
     float m = -INFINITY;
-    for (int k = 0; k < p.parts; ++k) m = fmaxf(m, p.lse[u + k * kRows]);
+    for (int k = 0; k < p.parts; ++k) m = fmaxf(m, p.stats[u + k * kRows].x);
     float acc[8] = {}, sum = 0.f;
     for (int k = 0; k < p.parts; ++k) {
-        const float w = __builtin_amdgcn_exp2f(p.lse[u + k * kRows] - m);
+        const float2 st = p.stats[u + k * kRows];
+        const float w = __builtin_amdgcn_exp2f(st.x - m);
         const f32x4 *x = reinterpret_cast<const f32x4 *>(p.part + (u + k * kRows) * D + c * 8);
         const f32x4 lo = x[0], hi = x[1];
-        sum += w;
+        sum += w * st.y;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             acc[e] = __builtin_fmaf(w, lo[e], acc[e]);
@@ -415,7 +429,7 @@ extern "C" int64_t ltxk_attention_workspace_bytes(int64_t batch, int64_t tokens_
 {
     if (batch <= 0 || tokens_q <= 0 || tokens_k <= 0 || heads <= 0 || head_dim <= 0) return 0;
     const FlashCut c = cut(batch * heads, tokens_q, tokens_k);
-    return 8 * c.rest * c.parts * kRows * (head_dim + 1) * 4;
+    return 8 * c.rest * c.parts * kRows * (head_dim + 2) * 4;
 }
 
 extern "C" int ltxk_attention(void *out, const void *q, int64_t q_bstride, int64_t q_tstride, const void *k,
@@ -465,7 +479,7 @@ extern "C" int ltxk_attention(void *out, const void *q, int64_t q_bstride, int64
     p.logits = static_cast<const uint16_t *>(logits);
     p.out = static_cast<uint16_t *>(out);
     p.part = static_cast<float *>(workspace);
-    p.lse = p.part + 8 * c.rest * c.parts * kRows * head_dim;
+    p.stats = reinterpret_cast<float2 *>(p.part + 8 * c.rest * c.parts * kRows * head_dim);
     p.qbs = q_bstride;
     p.kbs = k_bstride;
     p.vbs = v_bstride;

@@ -145,3 +145,20 @@ def test_attend_under_a_transform_and_a_mode():
     with FlopCounterMode(display=False) as counted:
         layer.attend(q[0], k[0], v[0], None)
     assert counted.get_total_flops() >= 2 * 2 * 70 * 256 * (70 + 70 + 256)
+
+
+@pytest.mark.parametrize("size", [2.0**10, 2.0**20, 2.0**26, 2.0**34, 2.0**100])
+@pytest.mark.parametrize("tk,sign", [(64, 1), (70, -1), (3000, 1)])
+def test_large_scores(size, tk, sign):
+    """Scores of either sign up to far past 2^31, in which the rounding of a scaled
+    score spans whole powers of two, with the largest of a row repeated over the
+    units of cut keys: softmax of them as in 64 bits, one-hot or the mean of equals."""
+    import ltxk
+
+    q = torch.zeros(1, 40, 128, device=DEV)
+    q[..., ::64] = size**0.5 * torch.linspace(1, 1.9, 40, device=DEV).view(1, 40, 1)
+    k = torch.zeros(1, tk, 128, device=DEV)
+    k[..., ::64] = sign * (torch.arange(tk, device=DEV) % 127 + 129).view(1, tk, 1) * size**0.5 / 256
+    v = torch.randn(1, tk, 128, device=DEV, generator=torch.Generator(device=DEV).manual_seed(tk))
+    q, k, v = (t.to(torch.bfloat16) for t in (q, k, v))
+    _check(q, k, v, 2, None, ltxk.attention(q, k, v, 2))
