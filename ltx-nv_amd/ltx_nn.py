@@ -93,15 +93,28 @@ def attention_grid_fits(batch: int, tokens: int, heads: int) -> bool:
     return batch <= 1 << 20 and -(-batch * heads // 8) * -(-tokens // 128) < (1 << 21) - 64
 
 
+def many_short_sequences(batch: int, tokens_q: int, tokens_k: int, heads: int, dim_head: int) -> bool:
+    """Shapes that torch's attention, in tiles of 16, runs faster than ltxk_attention in
+    its tiles of 128 queries and 64 keys.  Measured, torch (with the gate's launch) /
+    ltxk_attention, us, for batch * heads of 2048, 4096 and 8192:
+      heads of 64, 16 x 16 tokens: 10 / 12, 14 / 22, 21 / 42;  17 x 16: 15 / 12, -, 41 / 43;
+        16 x 17: 15 / 12, -, 40 / 43;
+      heads of 128, 32 x 16: 19 / 23, 33 / 41, 58 / 77;  40 x 16: 27 / 24, 47 / 44, 88 / 85;
+        32 x 17 and more: faster here too (20 x 17: 26 / 22, -, 88 / 74).
+    Up to 2048 the second launch costs the host more than is lost here."""
+    return tokens_k <= 16 and tokens_q <= dim_head // 4 and batch * heads > 2048
+
+
 def fused_attention_applies(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, heads: int, dim_head: int) -> bool:
     """Whether unmasked attention of token-major q over k, v runs on
     ltxk_attention: contiguous 16-byte aligned bf16 tensors on one ROCm device,
     heads of 64 or 128, keys of one batch item within the kernel's 32-bit
-    offsets, queries within its launch, no gradient to record and an
-    eager call."""
+    offsets, queries within its launch, not many_short_sequences, no gradient to
+    record and an eager call."""
     if not (dim_head in ltxk.ATTENTION_HEAD_DIMS and q.ndim == k.ndim == 3 and v.shape == k.shape
             and q.shape[0] == k.shape[0] and q.shape[2] == k.shape[2] == heads * dim_head and k.shape[1] > 0
-            and (k.shape[1] + 64) * k.shape[2] < 2**30 and attention_grid_fits(q.shape[0], q.shape[1], heads)):
+            and (k.shape[1] + 64) * k.shape[2] < 2**30 and attention_grid_fits(q.shape[0], q.shape[1], heads)
+            and not many_short_sequences(q.shape[0], q.shape[1], k.shape[1], heads, dim_head)):
         return False
     if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad) or not eager_call():
         return False

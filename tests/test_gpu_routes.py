@@ -199,3 +199,11 @@ def test_layers_of_an_attention_and_a_feed_forward(calls):
     ffn = ltx_nn.FeedForward(4096, 256).to(device=DEV, dtype=BF16).requires_grad_(False)
     ffn(torch.randn(1, 40, 4096, device=DEV).to(BF16))
     assert calls == {"linear": 1}
+
+
+def test_attend_of_many_short_sequences_keeps_torch(calls):
+    layer, q, k, v, gates = _attend(32, 64, tq=16, tk=16, b=65)
+    _close(layer.attend(q, k, v, gates), _want(layer, q, k, v, gates))
+    assert calls == {"sdpa": 1}
+    layer.attend(*(t[1:].contiguous() for t in (q, k, v, gates)))
+    assert calls == {"sdpa": 1, "attention": 1}

@@ -122,3 +122,12 @@ def test_calls_that_torch_watches_are_no_eager_calls():
         call(forward_ad.make_dual(x, x))
     assert len(seen) >= 7 and not any(seen)
     assert ltx_nn.eager_call()
+
+
+@pytest.mark.parametrize("batch,tq,tk,heads,dh,torchs", [
+    (65, 16, 16, 32, 64, True), (64, 16, 16, 32, 64, False), (65, 17, 16, 32, 64, False), (65, 16, 17, 32, 64, False),
+    (65, 32, 1, 32, 128, True), (65, 33, 1, 32, 128, False), (65, 32, 17, 32, 128, False), (4, 16, 16, 32, 64, False)])
+def test_many_short_sequences(batch, tq, tk, heads, dh, torchs):
+    import ltx_nn
+
+    assert ltx_nn.many_short_sequences(batch, tq, tk, heads, dh) == torchs
