@@ -327,13 +327,16 @@ def long_k_tiles(m: int, n: int, k: int) -> bool:
     shapes that leave the library's product to few compute units for a long K
     (256 x 256 output tiles, 256 at a time).  Measured, library / ltxk_linear, us:
       K 188160 x N 4096 (2048), M 128: 586 / 371 (404 / 192), 512: 1048 / 673
-        (742 / 363), 1024: 2100 / 1214 (1087 / 632);
-      K 16384 x N 4096, up to 64 tiles, M 256: 50 / 50, 512: 86 / 73, 1024: 124 / 121
-        (80 tiles and more: no faster, M 2048: 207 / 226);
+        (742 / 363), 1024: 2100 / 1214 (1087 / 632), 1280: 1807 / 1617, 1536:
+        1807 / 2112, 2048: 2067 / 2437 (2010 / 1242), 2560: (1598 / 1593), 4096:
+        3993 / 4739 (2072 / 2418);  K 65536 x N 4096, M 1280: 772 / 572, 2048: 767 / 863;
+      K 16384 x N 4096, M 128: 61 / 41, 256: 55 / 52, 512: 91 / 75, 1024: 130 / 126 (in
+        the text encoder, two blocks: 3864 / 3834 the whole call), 1280: 152 / 152,
+        2048: 207 / 226;
       K 8192 and less: the library's is faster (M 1008, N 2048: 46 / 49)."""
     if n % 8 or k % 64 or k < 16384 or max(m * k, n * k, m * n) >= 2**31:
         return False
-    return k >= 65536 or -(-m // 256) * -(-n // 256) <= 64
+    return -(-m // 256) * -(-n // 256) <= (80 if k >= 65536 else 64)
 
 
 def full_wave_rows(m: int, n: int, k: int) -> int:

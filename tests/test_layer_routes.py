@@ -131,3 +131,13 @@ def test_many_short_sequences(batch, tq, tk, heads, dh, torchs):
     import ltx_nn
 
     assert ltx_nn.many_short_sequences(batch, tq, tk, heads, dh) == torchs
+
+
+@pytest.mark.parametrize("m,n,k,own", [
+    (1024, 4096, 188160, True), (1280, 4096, 188160, True), (1281, 4096, 188160, False), (2560, 2048, 188160, True),
+    (2561, 2048, 188160, False), (1280, 4096, 65536, True), (1024, 4096, 16384, True), (1025, 4096, 16384, False),
+    (1280, 4096, 65472, False), (1024, 4096, 16320, False), (64, 4092, 16384, False)])
+def test_long_k_tiles(m, n, k, own):
+    import ltx_nn
+
+    assert ltx_nn.long_k_tiles(m, n, k) == own
