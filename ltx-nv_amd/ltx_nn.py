@@ -430,8 +430,20 @@ FEW_ROWS_MAX = 1 << 19
 
 
 def few_rows_widths(m: int, k: int, widths) -> bool:
-    """Whether ltxk_linear_layers takes layers of these widths over m rows of k: each
-    a multiple of 8, weights and outputs of fewer than 2^31 elements."""
+    """Whether layers of these widths over m rows of k go to ltxk_linear_layers: each a
+    multiple of 8, weights and outputs of fewer than 2^31 elements, K up to 6144, and
+    up to 160 of its tiles of 128 x 32 a layer (a launch takes 256 at a time, and what
+    it saves is a launch a layer).  Measured, layer by layer / ltxk_linear_layers,
+    device us:
+      x [256, 2048], N 2 x 2048 (128 tiles a layer): 19 / 13, 2 x 3072 (192): 21 / 25,
+        3 x 2560 (160): 31 / 25;  [126, 2048], 4 x 4096 (128): 38 / 27;
+      x [1024, 512], 3 x 576 (144): 18 / 12, 2 x 2048 (512): 14 / 23;  [4096, 128],
+        3 x 1024 (1024): 19 / 45;
+      x [80, 6144], 3 x 2048: 39 / 29, 3 x 4096: 54 / 55;  [64, 8192], 3 x 2048: 52 / 38,
+        2 x 2048: 35 / 36, 3 x 4096: 56 / 74, 8192 + 32: 39 / 72;  [32, 16384],
+        2 x 4096: 59 / 69."""
+    if k > 6144 or -(-m // 128) * sum(-(-n // 32) for n in widths) > 160 * len(widths):
+        return False
     return all(n % 8 == 0 and max(m, k) * n < 2**31 for n in widths)
 
 

@@ -59,11 +59,13 @@ def test_operand_kept_elsewhere_keeps_torch(name, where):
 
 
 @pytest.mark.parametrize("m,k,widths,taken", [
-    (1, 128, (8, 2**24 - 8), True), (1, 128, (8, 2**24), False), (4, 128, (2**24 + 8, 8), False),
-    (4096, 128, (2**19 - 8, 8), True), (4096, 128, (8, 2**19), False), (126, 2048, (2048, 2048, 2048, 32), True),
-    (126, 2048, (2048, 36), False)])
+    (1, 128, (8, 8), True), (1, 128, (8, 2**24), False), (4, 128, (2**24 + 8, 8), False),
+    (126, 2048, (2048, 2048, 2048, 32), True), (256, 2048, (2048, 2048, 2048, 32), True),
+    (128, 4096, (4096, 4096, 4096, 32), True), (126, 2048, (2048, 36), False),
+    (256, 2048, (2560, 2560), True), (256, 2048, (2568, 2560), False), (4096, 128, (160, 160), True),
+    (4096, 128, (1024, 1024, 1024), False), (80, 6144, (2048, 2048), True), (80, 6272, (2048, 2048), False)])
 def test_few_rows_widths(m, k, widths, taken):
-    """Layers that ltxk_linear_layers refuses keep torch's call."""
+    """Layers that ltxk_linear_layers refuses, and that it is slower on, keep torch's call."""
     import ltx_nn
 
     assert ltx_nn.few_rows_widths(m, k, widths) == taken
