@@ -126,8 +126,9 @@ class Embeddings1DConnector(torch.nn.Module):
             additive_mask = torch.zeros_like(additive_mask)
         pe = self._rope(b, s, hidden_states.device, hidden_states.dtype)
         x, pending = hidden_states.contiguous(), None
-        # a mask of zeros adds nothing to the scores: the blocks run unmasked
-        mask = None if self.num_registers else additive_mask
+        mask = additive_mask
+        if self.num_registers and mask.dtype == x.dtype and mask.shape[0] in (1, b) and mask.shape[1:] == (1, 1, s):
+            mask = None  # zeros that the attention takes add nothing to its scores: the blocks run unmasked
         for block in self.blocks:
             x, pending = block._run(x, pending, mask, pe, defer=True)
         if pending is None:

@@ -143,3 +143,35 @@ def test_long_k_tiles(m, n, k, own):
     import ltx_nn
 
     assert ltx_nn.long_k_tiles(m, n, k) == own
+
+
+@pytest.mark.parametrize("dtype,shape,dropped", [
+    (BF16, (2, 1, 1, 8), True), (BF16, (1, 1, 1, 8), True), (torch.float32, (2, 1, 1, 8), False),
+    (torch.bool, (2, 1, 1, 8), False), (BF16, (2, 3, 1, 8), False), (BF16, (2, 1, 8, 8), False),
+    (BF16, (2, 1, 5, 8), False), (BF16, (2, 1, 1, 1), False)])
+def test_connector_drops_only_masks_that_its_attention_takes(monkeypatch, dtype, shape, dropped):
+    """With registers every token is open: the blocks run unmasked, except under a
+    mask of a type or shape that the attention is to refuse (or to read another way)."""
+    import ltx_te
+    import ltxk
+
+    seen = []
+
+    class Block(torch.nn.Module):
+        def __init__(self):
+            super().__init__()
+            self.attn1 = torch.nn.Module()
+            self.attn1.heads = 2
+
+        def _run(self, x, pending, mask, pe, defer):
+            seen.append(mask)
+            return x, x
+
+    monkeypatch.setattr(ltxk, "add_norm_modulate", lambda x, f, eps: (x, x))
+    connector = ltx_te.Embeddings1DConnector(2, 16, 0, [16], 4, False, True)
+    connector.blocks.append(Block())
+    connector.learnable_registers.requires_grad_(False).zero_()
+    _, mask = connector(torch.zeros(2, 8, 32, dtype=BF16), torch.zeros(shape, dtype=dtype))
+    assert mask.shape == shape and mask.dtype == dtype
+    assert (seen[0] is None) == dropped
+    assert dropped or (seen[0].shape == shape and seen[0].dtype == dtype)
