@@ -110,13 +110,15 @@ def fused_attention_applies(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, h
     ltxk_attention: contiguous 16-byte aligned bf16 tensors on one ROCm device,
     heads of 64 or 128, keys of one batch item within the kernel's 32-bit
     offsets, queries within its launch, not many_short_sequences, no gradient to
-    record and an eager call."""
+    record, an eager call and no autocast to another type."""
     if not (dim_head in ltxk.ATTENTION_HEAD_DIMS and q.ndim == k.ndim == 3 and v.shape == k.shape
             and q.shape[0] == k.shape[0] and q.shape[2] == k.shape[2] == heads * dim_head and k.shape[1] > 0
             and (k.shape[1] + 64) * k.shape[2] < 2**30 and attention_grid_fits(q.shape[0], q.shape[1], heads)
             and not many_short_sequences(q.shape[0], q.shape[1], k.shape[1], heads, dim_head)):
         return False
     if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad) or not eager_call():
+        return False
+    if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.bfloat16:
         return False
     return all(t.is_cuda and t.device == q.device and t.dtype == torch.bfloat16 and t.is_contiguous()
                and t.data_ptr() % 16 == 0 for t in (q, k, v))

@@ -207,3 +207,18 @@ def test_attend_of_many_short_sequences_keeps_torch(calls):
     assert calls == {"sdpa": 1}
     layer.attend(*(t[1:].contiguous() for t in (q, k, v, gates)))
     assert calls == {"sdpa": 1, "attention": 1}
+
+
+def test_attend_under_autocast(calls):
+    """torch's attention casts to autocast's type: to float16 the call stays there
+    (and the gate refuses its result), to bfloat16 nothing changes."""
+    layer, q, k, v, gates = _attend(4, 64)
+    with torch.autocast("cuda", dtype=BF16):
+        _close(layer.attend(q, k, v, gates), _want(layer, q, k, v, gates))
+    assert calls == {"attention": 1}
+    with torch.autocast("cuda", dtype=torch.float16):
+        out = layer.attend(q, k, v, None)
+        with pytest.raises(RuntimeError):
+            layer.attend(q, k, v, gates)
+    assert out.dtype == torch.float16 and calls == {"attention": 1, "sdpa": 2}
+    _close(out, _want(layer, q, k, v))
