@@ -17,16 +17,22 @@ def _case(m, n, k, bias, seed=0):
 
 
 def _check(x, w, b, got):
-    """fp32 sums of k exact products move by at most k 2^-24 of the sum of their
-    sizes (in any order), the rounding to bf16 by 2^-8 of the result."""
+    """The rounding to bf16 moves a result by 2^-8 of it, and each of the k fp32
+    additions by 2^-24 of a partial sum.  Partial sums of independent signs stay
+    within 4 r, r the root of the summed squared products, and by Hoeffding's
+    inequality k independent roundings of at most 2^-24 4 r each add up to more than
+    6 sqrt(k) 2^-24 4 r for 3 results in 10^8."""
     k = x.shape[-1]
     for r in range(0, x.shape[0], 512):
         xr = x[r:r + 512].double()
-        want, size = xr @ w.double().T, xr.abs() @ w.double().abs().T
-        if b is not None:
-            want, size = want + b.double(), size + b.double().abs()
-        err = (got[r:r + 512].double() - want).abs()
-        assert bool((err <= want.abs() * 2.0**-8 + size * k * 2.0**-24 + 1e-30).all()), f"rows {r}.."
+        for c in range(0, w.shape[0], 512):
+            wc = w[c:c + 512].double()
+            want, square = xr @ wc.T, xr.square() @ wc.square().T
+            if b is not None:
+                want, square = want + b[c:c + 512].double(), square + b[c:c + 512].double().square()
+            err = (got[r:r + 512, c:c + 512].double() - want).abs()
+            bound = want.abs() * 2.0**-8 + square.sqrt() * (24 * k**0.5 * 2.0**-24) + 1e-30
+            assert bool((err <= bound).all()), f"rows {r}.. columns {c}..: {(err / bound).max().item():.3f}"
 
 
 @pytest.mark.parametrize("m,n,k,bias", [
@@ -39,6 +45,16 @@ def test_linear_matches_fp64(m, n, k, bias):
     import ltxk
 
     x, w, b = _case(m, n, k, bias)
+    _check(x, w, b, ltxk.linear(x, w, b))
+
+
+@pytest.mark.parametrize("m,n,bias", [(300, 6000, False), (130, 40, True)])
+def test_feature_projection_matches_fp64(m, n, bias):
+    """K 188160: 48 tiles in 5 parts with weight rows past 2^31 bytes, and one tile in
+    256 parts."""
+    import ltxk
+
+    x, w, b = _case(m, n, 188160, bias)
     _check(x, w, b, ltxk.linear(x, w, b))
 
 
