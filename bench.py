@@ -11,7 +11,7 @@ one full 48-block audio-video denoise step (fused kernels vs the reference's
 unfused eager PyTorch op sequence on the same GPU, with the GEMM/attention
 outputs supplied as pre-made tensors) and the host time to enqueue it;
 `full_step` and `guided_step` time whole denoise steps of the 48-block model
-(GEMMs and attention on PyTorch-ROCm).  `cpu_baseline` times the oracle's CPU
+(most GEMMs on PyTorch-ROCm, attention on ltxk_attention).  `cpu_baseline` times the oracle's CPU
 restatement of every config on the host.
 
 Timing: before the first kernel the GPU runs the headline kernel back to back
@@ -533,7 +533,7 @@ def bench_kernels(steps: int, warmup: int, only: set[str], settle_s: float = SET
         out.update([line("guide_step_video_eager", t, nbytes, {"config": "same, PyTorch-ROCm eager ops"})])
         del lat, vel, ts, nxt, den
 
-    # the V2A attention's key-split merge + head merge + per-head gate (ltx_nn.py:22-26,227-235): 8 chunk
+    # a key-split attention's merge + head merge + per-head gate (ltx_nn.py:22-26,227-235): 8 chunk
     # outputs of 126 audio queries x 32 heads x 64 and their log-sum-exps -> the gated token-major output
     if want("attn_combine"):
         parts, h_, t_, d_ = 8, 32, 126, 64

@@ -346,7 +346,7 @@ int ltxk_head_gate(void *out, const void *x, int64_t x_bstride, int64_t x_tstrid
  * of 8); lse element (b, c, h, t) likewise (fp32); out contiguous token-major
  * [batch*tokens, heads*head_dim]; parts a power of two up to 16.
  * Stands in for SDPA (ltx_nn.py:22-26,227) when the keys are split for few
- * queries over many keys (the V2A attention), and for the head merge and gate
+ * queries over many keys, and for the head merge and gate
  * after it (ltx_nn.py:228-235). */
 int ltxk_attn_combine(void *out, const void *part, int64_t part_bstride, int64_t part_cstride,
                       int64_t part_hstride, int64_t part_tstride, const float *lse, int64_t lse_bstride,

@@ -1,8 +1,8 @@
-// Combine of key-split attention: the V2A attention (a few hundred queries
-// over thousands of keys) runs PyTorch's flash kernel over the keys cut into
-// `parts` chunks (the chunks as extra batch items), which returns one output
-// and one log-sum-exp per chunk; this kernel merges them and applies the
-// per-head gate of the attention epilogue in the same pass:
+// Combine of key-split attention: where PyTorch's flash kernel runs a few
+// hundred queries over thousands of keys (heads that ltxk_attention does not
+// take), the keys are cut into `parts` chunks (the chunks as extra batch items),
+// and it returns one output and one log-sum-exp per chunk; this kernel merges
+// them and applies the per-head gate of the attention epilogue in the same pass:
 //
 //   w_c = exp(lse_c - max_c lse_c) / sum_c exp(lse_c - max_c lse_c)
 //   o   = round_bf16(sum_c w_c * part_c)                (fp32, one rounding)

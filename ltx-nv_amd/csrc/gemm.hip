@@ -4,7 +4,7 @@
 // pass.
 //
 // What bounds it: the card's power and, with it, the loads beside the products.
-// [1024, 188160] x [4096, 188160] takes 1214-1236 us, 1.28-1.30 PFLOP/s (the
+// [1024, 188160] x [4096, 188160] takes 1214-1266 us, 1.25-1.30 PFLOP/s (the
 // library's product, which leaves three of four compute units idle: 2100-2139 us,
 // 0.74-0.75), [512, 16384] x [4096, 16384] 73 (86).  On zeros, 8192^3 runs at
 // 1.72 PFLOP/s and 2.07 without its loads.  So:
@@ -53,12 +53,14 @@ __device__ __forceinline__ void tile_rows(const GemmParams &p, int t, int &m0, i
 // one chunk column, which a fragment read takes at a time, cover all banks.
 __device__ __forceinline__ int chunk_pos(int row, int c) { return c ^ ((row >> 1) & 7); }
 
-// 64 lanes x 16 bytes from memory straight to LDS at `lds` (through m0, which the
-// compiler sets anew before any use of its own).  In assembly because the
-// compiler, which cannot tell the buffers of a ring apart, would wait for every
-// load in flight before each LDS read; it has no output register, and its wait is
-// step_barrier's.  The wait states cover scalar operands that a vector instruction
-// has just written, which the compiler does not see the load read.
+// 64 lanes x 16 bytes from memory straight to LDS at `lds`, through m0.  In assembly
+// because the compiler, which cannot tell the buffers of a ring apart, would wait
+// for every load in flight before each LDS read; it has no output register, and its
+// wait is step_barrier's.  The wait states cover scalar operands that a vector
+// instruction has just written, which the compiler does not see the load read.  It
+// does not see m0 change either (a reserved register, whose clobber it ignores with
+// a warning): nothing else in these kernels may use m0, such as an LDS load builtin,
+// an indexed register or a message, and their assembly holds no other use.
 __device__ __forceinline__ void load_lds(const u32x4 &rsrc, uint32_t lds, uint32_t off, uint32_t soff)
 {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"

@@ -13,8 +13,8 @@ norm + layer interleave + token mask + projection scales is one
 ltxk_feature_norm pass; in the connector blocks every residual add is fused
 with the RMSNorm that follows it (the FFN residual with the next block's first
 norm, the last one with the output norm), q/k norm + RoPE, the attention head
-gate and GELU are the DiT's kernels.  Linear layers and attention are
-PyTorch-ROCm.
+gate and GELU are the DiT's kernels, and so are the attention and the linear
+layers that ltx_nn's rules name; the other linear layers are PyTorch-ROCm's.
 """
 
 from __future__ import annotations

@@ -1,6 +1,6 @@
 """Attention on PyTorch-ROCm as ltx_nn.sdpa runs it (GPU): the key-split form
-used for few queries over many keys (the V2A attention, 126 audio tokens over
-6144 video tokens) equals the softmax attention within the bf16 rounding of its
+used for few queries over many keys (126 tokens over 6144; in the model only for
+heads that ltxk_attention does not take) equals the softmax attention within the bf16 rounding of its
 result, on the token-major views the model passes and on contiguous inputs,
 against an fp32 evaluation of the formula and against PyTorch's own bf16
 attention."""
@@ -25,7 +25,7 @@ def test_key_split_attention_matches_softmax_attention(b, tq, tk, h, d, views):
     import ltx_nn
 
     g = torch.Generator(device=DEV).manual_seed(tq + tk)
-    if views:  # token-major projections viewed as (B, H, T, D), as Attention.forward passes them
+    if views:  # token-major projections viewed as (B, H, T, D), as Attention.attend passes them
         q, k, v = (torch.randn(b, t, h * d, device=DEV, generator=g).to(torch.bfloat16).view(b, t, h, d)
                    .transpose(1, 2) for t in (tq, tk, tk))
     else:
@@ -58,9 +58,9 @@ def test_masked_or_many_query_attention_keeps_the_library_path():
 
 
 def test_key_split_attention_with_the_gate_in_the_combine():
-    """Attention.attend on the V2A shape (126 audio queries over 6144 video keys,
-    32 heads x 64, gated): the key-split merge, head merge and per-head gate in
-    one ltxk_attn_combine pass equal the unfused sequence (merge, then
+    """The pieces of the key-split form on 126 queries over 6144 keys, 32 heads x 64,
+    gated: the key-split merge, head merge and per-head gate in one
+    ltxk_attn_combine pass equal the unfused sequence (merge, then
     ltxk_head_gate) bit for bit, and 2*sigmoid(logit) * softmax attention in
     fp32 within the bf16 rounding of the result."""
     import ltx_nn

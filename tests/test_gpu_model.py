@@ -7,8 +7,8 @@ optional metadata keys gets (no cross-attention AdaLN: 6-row tables and an ungat
 text cross-attention; no per-head attention gates; biased video FFN projections; the
 fp32 RoPE grid; no keyframe embedding).
 
-GEMMs and attention run in bf16 on PyTorch-ROCm here and in fp32/bf16 on the CPU in
-the reference, so the check is statistical: the fused bf16 result must be as close
+GEMMs and attention run in bf16 on the GPU here and in fp32/bf16 on the CPU in the
+reference, so the check is statistical: the fused bf16 result must be as close
 to the reference's fp32 result as the reference's own bf16 run is (relative L2 within
 1.5x of it, and cosine >= 0.999), which a wrong AdaLN row, a swapped shift/scale, a
 missing residual or a wrong mask would break by orders of magnitude."""

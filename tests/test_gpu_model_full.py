@@ -7,8 +7,8 @@ Shape: video 16x16x24 latent grid = 6144 tokens x 4096 (32 heads x 128), audio
 audio), FFN 4x, 2 blocks, weights N(0, 0.02^2) bf16 (seed 123), sigma 0.5.
 This composes the forms the model takes only at this size: the streaming row
 kernels on 4096/2048-wide rows, the compact 56-row RoPE tables, the two-row
-q/k kernel, unpaired A2V/V2A q/k with 6144 and 126 tokens, the key-split V2A
-attention (126 queries over 6144 keys) and the audio side stream.
+q/k kernel, unpaired A2V/V2A q/k with 6144 and 126 tokens, the V2A attention with
+its keys cut (126 queries over 6144 keys) and the audio side stream.
 
 Criteria (as tests/test_gpu_model.py): the eager fp32 run is the target, the
 eager bf16 run (the reference's rounding after every op) gives the spread;
@@ -181,7 +181,7 @@ def test_48_blocks_against_eager(batch):
     restatement (ltx_dit.py:354-378 block by block), fp32 target and eager-bf16
     spread as above.  B=4 is the guidance batch with STG at block 28 and the
     modality-isolated pass (the reference's run_all.py settings).  The V2A
-    attention (32 queries over 2048 keys) takes the key-split path."""
+    attention (32 queries over 2048 keys) runs with its keys cut."""
     import ltx_dit
 
     cfg, model = _model(layers=48)

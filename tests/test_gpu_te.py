@@ -5,8 +5,8 @@ EmbeddingsProcessor.process_hidden_states on a small configuration: 4 layers of
 64, video connector 2x64 gated, audio 2x32, 2 blocks, 4 registers, B=2 with
 left padding).
 
-Projections and attention run in bf16 on PyTorch-ROCm here and in fp32/bf16 on
-the CPU in the reference, so the module check is statistical, as for LTXModel:
+Projections and attention run in bf16 on the GPU here and in fp32/bf16 on the
+CPU in the reference, so the module check is statistical, as for LTXModel:
 relative L2 to the fp32 reference within 1.5x of the reference's own bf16 run,
 cosine >= 0.999."""
 
