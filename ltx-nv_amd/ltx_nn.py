@@ -18,6 +18,7 @@ import numpy
 import torch
 import torch.nn.functional as F
 from torch.autograd import forward_ad
+from torch.compiler import is_compiling
 from torch.nn.attention import SDPBackend, sdpa_kernel
 from torch.nn.modules.module import _has_any_global_hook
 
@@ -35,10 +36,11 @@ def rms_norm(x: torch.Tensor, eps: float = 1e-6, weight: torch.Tensor | None = N
 def sdpa(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask: torch.Tensor | None = None) -> torch.Tensor:
     """q,k,v: (B, H, T, D); PyTorch-ROCm attention with the reference's backend order (ltx_nn.py:22-26).
 
-    Few queries over many keys (the V2A attention: 126 audio tokens over 6144
-    video tokens) leave the flash kernel a handful of query tiles, so it runs
-    on a few CUs; that shape is split over the keys instead (key_split_applies,
-    key_split_partials) and merged by ltxk_attn_combine."""
+    Few queries over many keys (126 audio tokens over 6144 video tokens) leave the
+    flash kernel a handful of query tiles, so it runs on a few CUs; that shape is
+    split over the keys instead (key_split_applies, key_split_partials) and merged
+    by ltxk_attn_combine.  Attention comes here with what ltxk_attention does not
+    take (fused_attention_applies)."""
     if key_split_applies(q, k, mask):
         b, h, tq, d = q.shape
         merged = ltxk.attn_combine(*key_split_partials(q, k, v, KEY_SPLIT_PARTS), KEY_SPLIT_PARTS)
@@ -78,12 +80,16 @@ def key_split_partials(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, parts:
     return out, lse
 
 
+_dispatch_modes, _transform = torch._C._len_torch_dispatch_stack, torch._C._functorch.peek_interpreter_stack
+_tracing = torch._C._is_tracing
+
+
 def eager_call() -> bool:
-    """Whether operations just run as they are called: no tracer, function transform,
-    forward-mode derivative or dispatch mode is to see them.  The ltxk entry points
-    bypass torch's dispatcher, so calls that one watches keep torch's operations."""
-    return not (torch._C._len_torch_dispatch_stack() or torch._C._is_tracing() or forward_ad._current_level >= 0
-                or torch._C._functorch.peek_interpreter_stack() is not None or torch.compiler.is_compiling())
+    """Whether operations just run as they are called: no compiler, tracer, function
+    transform, forward-mode derivative or dispatch mode is to see them.  The ltxk entry
+    points bypass torch's dispatcher, so calls that one watches keep torch's operations."""
+    return not (is_compiling() or _dispatch_modes() or _tracing() or forward_ad._current_level >= 0
+                or _transform() is not None)
 
 
 def attention_grid_fits(batch: int, tokens: int, heads: int) -> bool:
@@ -111,17 +117,20 @@ def fused_attention_applies(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, h
     heads of 64 or 128, keys of one batch item within the kernel's 32-bit
     offsets, queries within its launch, not many_short_sequences, no gradient to
     record, an eager call and no autocast to another type."""
-    if not (dim_head in ltxk.ATTENTION_HEAD_DIMS and q.ndim == k.ndim == 3 and v.shape == k.shape
-            and q.shape[0] == k.shape[0] and q.shape[2] == k.shape[2] == heads * dim_head and k.shape[1] > 0
-            and (k.shape[1] + 64) * k.shape[2] < 2**30 and attention_grid_fits(q.shape[0], q.shape[1], heads)
-            and not many_short_sequences(q.shape[0], q.shape[1], k.shape[1], heads, dim_head)):
+    if dim_head not in ltxk.ATTENTION_HEAD_DIMS or not q.ndim == k.ndim == 3 or not eager_call():
         return False
-    if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad) or not eager_call():
+    (b, tq, d), (kb, tk, kd) = q.shape, k.shape
+    if not (b == kb and d == kd == heads * dim_head and v.shape == k.shape and 0 < tk and (tk + 64) * d < 2**30
+            and attention_grid_fits(b, tq, heads)) or many_short_sequences(b, tq, tk, heads, dim_head):
         return False
     if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.bfloat16:
         return False
-    return all(t.is_cuda and t.device == q.device and t.dtype == torch.bfloat16 and t.is_contiguous()
-               and t.data_ptr() % 16 == 0 for t in (q, k, v))
+    device = q.get_device()
+    for t in (q, k, v):
+        if not (t.is_cuda and t.get_device() == device and t.dtype == torch.bfloat16 and t.is_contiguous()
+                and t.data_ptr() % 16 == 0) or (t.requires_grad and torch.is_grad_enabled()):
+            return False
+    return True
 
 
 # ---------------------------------------------------------------------------
@@ -346,12 +355,17 @@ def full_wave_rows(m: int, n: int, k: int) -> int:
     of 256 x 256, where few rows are left past them: those then go in a launch of
     their own, because the library gives them a whole further wave, or other tiles
     to all of it.  0: one launch.  Measured, one launch / two, us, N x K:
-      4096 x 4096, M 4160: 142 / 103, 4290: 137 / 107, 4800: 146 / 120, 8580: 221 / 201,
-        17160: 433 / 383;  4096 x 2048, M 4290: 83 / 60, 12500: 230 / 154;
-      16384 x 4096, M 4290: 433 / 383, 4800: 574 / 430, 17160: 1517 / 1524;
-      4096 x 16384, M 4290: 840 / 396, 8448: 1181 / 743, 17160: 1576 / 1525.
-    Above 768 rows the two are less often apart, and once the other way (4096 x 16384,
-    1769 rows past 4096: 584 / 746; 16384 x 4096, 808 past 8192: 790 / 812)."""
+      4096 x 4096, M 4160: 131 / 104, 4290: 131 / 110, 4800: 141 / 122, 8580: 221 / 205,
+        12500: 388 / 289, 24676: 657 / 548;  4096 x 2048, M 4290: 78 / 60, 12500: 223 / 156;
+      4096 x 8192, M 4290: 240 / 204;  4096 x 16384, M 4290: 844 / 401, 8448: 1198 / 760,
+        24776: 2386 / 2196;  4096 x 32768, M 4290: 1579 / 857;
+      8192 x 2048, M 4352: 145 / 117, 8900: 222 / 219;  8192 x 4096, M 4100: 305 / 192,
+        4600: 229 / 218, 8892: 412 / 403, 17084: 883 / 761;  8192 x 16384, M 4200: 1207 / 772;
+      16384 x 2048, M 4290: 253 / 215;  16384 x 4096, M 4290: 427 / 391, 4800: 572 / 438,
+        8892: 928 / 791, 17084: 1609 / 1504, 24776: 2207 / 2176.
+    Above 768 rows the two are less often apart, and three times the other way (4096 x
+    16384, 1769 rows past 4096: 584 / 746; 16384 x 4096, 808 past 8192: 790 / 812, 776
+    past 16384: 1517 / 1524)."""
     across = -(-n // 256)
     if n < 4096 or not 2048 <= k < 65536 or across > 64 or 256 % across:
         return 0
@@ -362,12 +376,13 @@ def full_wave_rows(m: int, n: int, k: int) -> int:
 
 def _plain_input(x: torch.Tensor) -> bool:
     """Whether the ltxk products can read x: contiguous aligned bf16 on a ROCm
-    device, no autocast, no gradient to record, an eager call."""
+    device, no autocast, no gradient to record, an eager call without module hooks."""
     return x.is_cuda and x.dtype == torch.bfloat16 and eager_call() and x.is_contiguous() and x.data_ptr() % 16 == 0 \
-        and x.numel() > 0 and not (torch.is_grad_enabled() and x.requires_grad) and not torch.is_autocast_enabled("cuda")
+        and x.numel() > 0 and not (x.requires_grad and torch.is_grad_enabled()) \
+        and not torch.is_autocast_enabled("cuda") and not _has_any_global_hook()
 
 
-_OWN_ATTRIBUTES = {"forward", "weight", "bias"}  # set on a layer itself, these come before its class and parameters
+_PLAIN = (torch.nn.Parameter, torch.Tensor)
 
 
 def _plain_layer(layer: torch.nn.Linear, x: torch.Tensor) -> tuple | None:
@@ -377,18 +392,20 @@ def _plain_layer(layer: torch.nn.Linear, x: torch.Tensor) -> tuple | None:
     out_features of them.  Reads the module's dictionaries: its attribute lookup
     costs more than the rest (`project` over four layers takes the host 30 us with
     it, 16 without)."""
-    if type(layer) is not torch.nn.Linear or layer._forward_hooks or layer._forward_pre_hooks \
-            or _OWN_ATTRIBUTES & layer.__dict__.keys() or _has_any_global_hook():
+    own = layer.__dict__
+    if type(layer) is not torch.nn.Linear or own["_forward_hooks"] or own["_forward_pre_hooks"] \
+            or "forward" in own or "weight" in own or "bias" in own:  # attributes come before class and parameters
         return None
-    params = layer._parameters
-    w, b = params.get("weight"), params.get("bias")
-    n = layer.out_features
-    if w is None or "bias" not in params or w.shape != (n, x.shape[-1]) or (b is not None and b.shape != (n,)):
+    params = own["_parameters"]
+    w, b, n = params.get("weight"), params.get("bias", False), own["out_features"]
+    if w is None or b is False:  # kept elsewhere
         return None
-    for t in (w, b):
-        if t is not None and not (type(t) in (torch.nn.Parameter, torch.Tensor) and t.get_device() == x.get_device()
-                                  and t.dtype == torch.bfloat16 and t.is_contiguous() and t.data_ptr() % 16 == 0
-                                  and not (t.requires_grad and torch.is_grad_enabled())):
+    if w.shape != (n, x.shape[-1]) or (b is not None and b.shape != (n,)):
+        return None
+    device, bf16 = x.get_device(), torch.bfloat16
+    for t in (w,) if b is None else (w, b):
+        if not (type(t) in _PLAIN and t.get_device() == device and t.dtype == bf16 and t.is_contiguous()
+                and t.data_ptr() % 16 == 0) or (t.requires_grad and torch.is_grad_enabled()):
             return None
     return w, b
 
@@ -444,9 +461,14 @@ def few_rows_widths(m: int, k: int, widths) -> bool:
       x [80, 6144], 3 x 2048: 39 / 29, 3 x 4096: 54 / 55;  [64, 8192], 3 x 2048: 52 / 38,
         2 x 2048: 35 / 36, 3 x 4096: 56 / 74, 8192 + 32: 39 / 72;  [32, 16384],
         2 x 4096: 59 / 69."""
-    if k > 6144 or -(-m // 128) * sum(-(-n // 32) for n in widths) > 160 * len(widths):
+    if k > 6144:
         return False
-    return all(n % 8 == 0 and max(m, k) * n < 2**31 for n in widths)
+    tiles = 0
+    for n in widths:
+        if n % 8 or max(m, k) * n >= 2**31:
+            return False
+        tiles += (n + 31) // 32
+    return -(-m // 128) * tiles <= 160 * len(widths)
 
 
 def project(x: torch.Tensor, *layers: torch.nn.Linear | None) -> list:
@@ -543,7 +565,8 @@ class Attention(torch.nn.Module):
             if mask.ndim == 3:
                 mask = mask.unsqueeze(1)
         if perturbation_mask is None and key_split_applies(q4, k4, mask):
-            # key-split attention: its merge, the head merge and the gate in one pass
+            # key-split attention (of heads that ltxk_attention does not take): its merge, the
+            # head merge and the gate in one pass
             part, lse = key_split_partials(q4, k4, v4, KEY_SPLIT_PARTS)
             return self.to_out(ltxk.attn_combine(part, lse, KEY_SPLIT_PARTS, gates))
         attn = sdpa(q4, k4, v4, mask)  # (B, H, T, D) view
