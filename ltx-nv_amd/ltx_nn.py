@@ -337,17 +337,28 @@ def long_k_tiles(m: int, n: int, k: int) -> bool:
     """Whether a product of (m, k) and (n, k) matrices goes to ltxk_linear: the
     shapes that leave the library's product to few compute units for a long K
     (256 x 256 output tiles, 256 at a time).  Measured, library / ltxk_linear, us:
-      K 188160 x N 4096 (2048), M 128: 586 / 371 (404 / 192), 512: 1048 / 673
-        (742 / 363), 1024: 2100 / 1214 (1087 / 632), 1280: 1807 / 1617, 1536:
-        1807 / 2112, 2048: 2067 / 2437 (2010 / 1242), 2560: (1598 / 1593), 4096:
-        3993 / 4739 (2072 / 2418);  K 65536 x N 4096, M 1280: 772 / 572, 2048: 767 / 863;
-      K 16384 x N 4096, M 128: 61 / 41, 256: 55 / 52, 512: 91 / 75, 1024: 130 / 126 (in
-        the text encoder, two blocks: 3864 / 3834 the whole call), 1280: 152 / 152,
-        2048: 207 / 226;
+      K 188160 x N 4096 (2048), M 8: 275 / 337 (358 / 182), 24: 671 / 345, 64: 616 / 352,
+        128: 586 / 371 (404 / 192), 512: 1048 / 673 (742 / 363), 1024: 2100 / 1214
+        (1087 / 632), 1280: 1807 / 1617, 1536: 1807 / 2112, 2048: 2067 / 2437 (2010 /
+        1242), 2560: (1598 / 1593), 4096: 3993 / 4739 (2072 / 2418);
+      K 65536 x N 4096, M 8: 116 / 122, 1280: 772 / 572, 2048: 767 / 863;  x N 16384,
+        M 24: 382 / 470, 64: 467 / 480, 96: 466 / 490;
+      K 32768 x N 3072, M 16: 37 / 46, 24: 73 / 49;  x N 8192, M 32: 100 / 123, 65: 200 / 134;
+      K 16384 x N 4096, M 33: 30 / 34, 64: 37 / 36, 65: 40 / 37, 128: 61 / 41, 256: 55 / 52,
+        512: 91 / 75, 1024: 130 / 126 (in the text encoder, two blocks: 3864 / 3834 the
+        whole call), 1280: 152 / 152, 2048: 207 / 226;  x N 8192, M 65: 57 / 66;
       K 8192 and less: the library's is faster (M 1008, N 2048: 46 / 49)."""
     if n % 8 or k % 64 or k < 16384 or max(m * k, n * k, m * n) >= 2**31:
         return False
-    return -(-m // 256) * -(-n // 256) <= (80 if k >= 65536 else 64)
+    if m < 24:
+        most = 8 if k >= 32768 else 2
+    elif m <= 64:
+        most = 20 if k >= 32768 else 2
+    elif m <= 128:
+        most = 32 if k >= 32768 else 16
+    else:
+        most = 80 if k >= 65536 else 64
+    return -(-m // 256) * -(-n // 256) <= most
 
 
 def full_wave_rows(m: int, n: int, k: int) -> int:

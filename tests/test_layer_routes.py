@@ -138,6 +138,9 @@ def test_many_short_sequences(batch, tq, tk, heads, dh, torchs):
 @pytest.mark.parametrize("m,n,k,own", [
     (1024, 4096, 188160, True), (1280, 4096, 188160, True), (1281, 4096, 188160, False), (2560, 2048, 188160, True),
     (2561, 2048, 188160, False), (1280, 4096, 65536, True), (1024, 4096, 16384, True), (1025, 4096, 16384, False),
+    (23, 2048, 188160, True), (23, 4096, 188160, False), (24, 4096, 188160, True), (64, 5376, 32768, False),
+    (65, 5376, 32768, True), (128, 8448, 32768, False), (129, 8448, 32768, True), (64, 4096, 16384, False),
+    (65, 4096, 16384, True), (64, 512, 16384, True), (128, 4352, 16384, False), (129, 4352, 16384, True),
     (1280, 4096, 65472, False), (1024, 4096, 16320, False), (64, 4092, 16384, False)])
 def test_long_k_tiles(m, n, k, own):
     import ltx_nn
