@@ -428,8 +428,8 @@ def linear(layer: torch.nn.Linear, x: torch.Tensor) -> torch.Tensor:
         return layer(x)
     k, n = x.shape[-1], layer.out_features
     m = x.numel() // max(k, 1)
-    own = long_k_tiles(m, n, k)
-    main = 0 if own else full_wave_rows(m, n, k)
+    own = k >= 16384 and long_k_tiles(m, n, k)
+    main = 0 if own or m <= 4096 else full_wave_rows(m, n, k)
     if (own or main) and _plain_input(x):
         plain = _plain_layer(layer, x)
         if plain is not None:
@@ -485,10 +485,12 @@ def few_rows_widths(m: int, k: int, widths) -> bool:
 def project(x: torch.Tensor, *layers: torch.nn.Linear | None) -> list:
     """[layer(x) for each layer], None for None, in one launch where x is small."""
     real = [layer for layer in layers if layer is not None]
-    if 2 <= len(real) <= ltxk.MAX_LINEAR_LAYERS and x.numel() <= FEW_ROWS_MAX and x.shape[-1] % 128 == 0 \
+    size, k = x.numel(), x.shape[-1]
+    if 2 <= len(real) <= ltxk.MAX_LINEAR_LAYERS and 0 < size <= FEW_ROWS_MAX and k % 128 == 0 \
+            and few_rows_widths(size // k, k, [i.out_features if type(i) is torch.nn.Linear else 1 for i in real]) \
             and _plain_input(x):
-        plain, k = [_plain_layer(layer, x) for layer in real], x.shape[-1]
-        if None not in plain and few_rows_widths(x.numel() // k, k, [w.shape[0] for w, _ in plain]):
+        plain = [_plain_layer(layer, x) for layer in real]
+        if None not in plain:
             weights, biases = zip(*plain)
             done = iter(ltxk._launch_layers(x, weights, biases))
             return [None if layer is None else next(done) for layer in layers]

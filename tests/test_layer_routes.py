@@ -75,16 +75,13 @@ def test_few_rows_of_a_huge_layer_keep_torch(monkeypatch):
     import ltx_nn
     import ltxk
 
-    class Huge(torch.nn.Module):  # stands for a layer of 2^24 + 8 rows of 128, which has no memory here
-        def forward(self, x):
-            return x.new_zeros(x.shape[0], 8)
-
-    layers = [Huge(), Huge()]
-    weight = torch.empty(2**24 + 8, 128, dtype=BF16, device="meta")
     monkeypatch.setattr(ltx_nn, "_plain_input", lambda x: True)
-    monkeypatch.setattr(ltx_nn, "_plain_layer", lambda layer, x: (weight, None))
-    monkeypatch.setattr(ltxk, "_launch_layers", lambda *a: pytest.fail("launched"))
-    assert [y.shape for y in ltx_nn.project(torch.zeros(2, 128, dtype=BF16), *layers)] == [(2, 8)] * 2
+    monkeypatch.setattr(ltxk, "_launch_layers", lambda *a: ["launched"] * 2)
+    x = torch.zeros(2, 128, dtype=BF16, device="meta")
+    for n, taken in ((64, True), (2**24 + 8, False)):
+        layers = [torch.nn.Linear(128, n, dtype=BF16, device="meta").requires_grad_(False) for _ in range(2)]
+        got = ltx_nn.project(x, *layers)
+        assert got == ["launched"] * 2 if taken else [y.shape for y in got] == [(2, n)] * 2
 
 
 @pytest.mark.parametrize("batch,tokens,heads,fits", [
